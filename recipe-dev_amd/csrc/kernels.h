@@ -87,10 +87,14 @@ size_t matvec_lds_bytes(int fmt, int xtype, int M, int cols);
 LaunchShape plan_fused(int fmt, int64_t rows, int64_t cols, int cus, bool glu, bool norm);
 hipError_t launch_matvec_fused(int fmt, const MvParams& p, const LaunchShape& s, hipStream_t stream);
 
-// Matrix-core product for 1 <= M <= 32 activation rows (quantized formats).
-hipError_t launch_matvec_mfma(int fmt, int xtype, int M, const MvParams& p, int cus, hipStream_t stream,
+// Matrix-core product for 1 <= M <= 32 fp16 activation rows (quantized formats).
+hipError_t launch_matvec_mfma(int fmt, int M, const MvParams& p, int cus, hipStream_t stream,
                               hipEvent_t ev0 = nullptr, hipEvent_t ev1 = nullptr);
-size_t mfma_lds_bytes(int fmt, int xtype, int M, int64_t rows, int cus);
+// fp32 activations on the matrix cores (mfma_f32.hip), any count of rows whose
+// activations span less than 4 GiB.
+hipError_t launch_matvec_f32(int fmt, const MvParams& p, int M, int cus, hipStream_t stream, hipEvent_t ev0 = nullptr,
+                             hipEvent_t ev1 = nullptr);
+size_t mfma_lds_bytes(int fmt, int M, int64_t rows, int cus);
 
 // recipe's int(8) sum (int8.hip): Q8 activation records of `step` (32 or 256)
 // inputs, v_dot4_i32_i8 block dots, recipe's fp32 order. y[m*ldy + n] for

@@ -1,5 +1,5 @@
-// Small-M quantized products on the matrix cores: launch planning and the
-// fp16-activation kernels (the kernels themselves are in mfma_impl.h).
+// Quantized products of fp16 activations on the matrix cores: launch planning
+// (the kernels are in mfma_rt.h and mfma_impl.h).
 #include "mfma_impl.h"
 #include "mfma_rt.h"
 
@@ -128,10 +128,10 @@ static hipError_t launch_mfma_sk(const MvParams& p, int M, uint32_t x_bytes, hip
 }
 
 template <int FMT>
-static size_t lds_of(bool f32, bool two, int W) {
-    if (W == 1 && (f32 || two)) W = 2;  // as launch_mfma_w
-#define RQ_LDS(NT, XF) (W == 1 ? MfmaLds<FMT, NT, XF, 1>::TOTAL : W == 2 ? MfmaLds<FMT, NT, XF, 2>::TOTAL : MfmaLds<FMT, NT, XF, 4>::TOTAL)
-    return two ? (f32 ? RQ_LDS(2, true) : RQ_LDS(2, false)) : (f32 ? RQ_LDS(1, true) : RQ_LDS(1, false));
+static size_t lds_of(bool two, int W) {
+    if (W == 1 && two) W = 2;  // as launch_mfma_w
+#define RQ_LDS(NT) (W == 1 ? MfmaLds<FMT, NT, 1>::TOTAL : W == 2 ? MfmaLds<FMT, NT, 2>::TOTAL : MfmaLds<FMT, NT, 4>::TOTAL)
+    return two ? RQ_LDS(2) : RQ_LDS(1);
 #undef RQ_LDS
 }
 
@@ -150,43 +150,36 @@ static int mfma_waves(int64_t rows, int cus) {
     return 1;
 }
 
-size_t mfma_lds_bytes(int fmt, int xtype, int M, int64_t rows, int cus) {
-    const bool f32 = xtype == X_F32, two = M > 16;
-    if (!two && !f32) {
+size_t mfma_lds_bytes(int fmt, int M, int64_t rows, int cus) {
+    const bool two = M > 16;
+    if (!two) {
         const size_t sk = fmt == Q4_0 ? SkLds<Q4_0>::TOTAL : fmt == Q4_K ? SkLds<Q4_K>::TOTAL
                         : fmt == Q8_0 ? SkLds<Q8_0>::TOTAL : fmt == Q6_K ? SkLds<Q6_K>::TOTAL : 0;
         if (sk) return sk;  // (the larger of the two forms is below the LDS limit either way)
     }
     const int W = mfma_waves(rows, cus);
     switch (fmt) {
-        case Q4_0: return lds_of<Q4_0>(f32, two, W);
-        case Q4_K: return lds_of<Q4_K>(f32, two, W);
-        case Q8_0: return lds_of<Q8_0>(f32, two, W);
-        case Q6_K: return lds_of<Q6_K>(f32, two, W);
+        case Q4_0: return lds_of<Q4_0>(two, W);
+        case Q4_K: return lds_of<Q4_K>(two, W);
+        case Q8_0: return lds_of<Q8_0>(two, W);
+        case Q6_K: return lds_of<Q6_K>(two, W);
         default: return 0;
     }
 }
 
-// fp32 activations (mfma_f32.hip: built without the matrix-core VGPR form,
-// which the per-block power-of-two epilogue of that path does not compile under).
-hipError_t launch_mfma_f32(int fmt, bool two, int W, const MvParams& p, int M, uint32_t x_bytes, hipStream_t stream,
-                           hipEvent_t ev0, hipEvent_t ev1);
-
 template <int FMT>
-static hipError_t launch_mfma_fmt(int xtype, int W, const MvParams& p, int M, uint32_t x_bytes, hipStream_t stream,
-                                  hipEvent_t ev0, hipEvent_t ev1) {
-    if (xtype == X_F32) return launch_mfma_f32(FMT, M > 16, W, p, M, x_bytes, stream, ev0, ev1);
-    if (M > 16) return launch_mfma_w<FMT, 2, false>(W, p, M, x_bytes, stream, ev0, ev1);
-    return launch_mfma_w<FMT, 1, false>(W, p, M, x_bytes, stream, ev0, ev1);
+static hipError_t launch_mfma_fmt(int W, const MvParams& p, int M, uint32_t x_bytes, hipStream_t stream, hipEvent_t ev0,
+                                  hipEvent_t ev1) {
+    if (M > 16) return launch_mfma_w<FMT, 2>(W, p, M, x_bytes, stream, ev0, ev1);
+    return launch_mfma_w<FMT, 1>(W, p, M, x_bytes, stream, ev0, ev1);
 }
 
-hipError_t launch_matvec_mfma(int fmt, int xtype, int M, const MvParams& p, int cus, hipStream_t stream,
+hipError_t launch_matvec_mfma(int fmt, int M, const MvParams& p, int cus, hipStream_t stream,
                               hipEvent_t ev0, hipEvent_t ev1) {
     if (M < 1 || M > 32) return hipErrorInvalidValue;
-    const size_t esize = xtype == X_F32 ? 4 : 2;
-    const int64_t x_bytes = ((int64_t)(M - 1) * p.ldx + p.K) * (int64_t)esize;
+    const int64_t x_bytes = ((int64_t)(M - 1) * p.ldx + p.K) * 2;
     if (x_bytes >= (int64_t)kOobOffset) return hipErrorInvalidValue;
-    // fp16 activations: the streaming form, unless its scale table does not
+    // The streaming form, unless its scale table does not
     // fit (K ranges longer than it holds) or RQMV_MFMA_RT=0 asks for the
     // staged forms below.
     const char* rt_env = getenv("RQMV_MFMA_RT");
@@ -194,7 +187,7 @@ hipError_t launch_matvec_mfma(int fmt, int xtype, int M, const MvParams& p, int 
     // whose waves read their activation fragments from the caches, measured
     // faster: Q4_K 14336->4096 at 16 rows 26.4 -> 24.1 us)
     const bool long_few = M <= 16 && p.K > 8192 && (p.rows + 15) / 16 < (int64_t)2 * cus;
-    if (xtype == X_F16 && !(rt_env && *rt_env == '0') && !(long_few && !(rt_env && *rt_env == '1'))) {
+    if (!(rt_env && *rt_env == '0') && !(long_few && !(rt_env && *rt_env == '1'))) {
         hipError_t e = hipErrorInvalidValue;
         switch (fmt) {
             case Q4_0: e = launch_rt_fmt<Q4_0>(p, M, (uint32_t)x_bytes, cus, stream, ev0, ev1); break;
@@ -211,7 +204,7 @@ hipError_t launch_matvec_mfma(int fmt, int xtype, int M, const MvParams& p, int 
     // RQMV_MFMA_SK=0/1 forces either.
     const char* sk_env = getenv("RQMV_MFMA_SK");
     const bool sk = sk_env && *sk_env ? *sk_env != '0' : (p.rows + 15) / 16 <= (int64_t)4 * cus;
-    if (M <= 16 && xtype == X_F16 && sk) {
+    if (M <= 16 && sk) {
         switch (fmt) {
             case Q4_0: return launch_mfma_sk<Q4_0>(p, M, (uint32_t)x_bytes, stream, ev0, ev1);
             case Q4_K: return launch_mfma_sk<Q4_K>(p, M, (uint32_t)x_bytes, stream, ev0, ev1);
@@ -222,10 +215,10 @@ hipError_t launch_matvec_mfma(int fmt, int xtype, int M, const MvParams& p, int 
     }
     const int W = mfma_waves(p.rows, cus);
     switch (fmt) {
-        case Q4_0: return launch_mfma_fmt<Q4_0>(xtype, W, p, M, (uint32_t)x_bytes, stream, ev0, ev1);
-        case Q4_K: return launch_mfma_fmt<Q4_K>(xtype, W, p, M, (uint32_t)x_bytes, stream, ev0, ev1);
-        case Q8_0: return launch_mfma_fmt<Q8_0>(xtype, W, p, M, (uint32_t)x_bytes, stream, ev0, ev1);
-        case Q6_K: return launch_mfma_fmt<Q6_K>(xtype, W, p, M, (uint32_t)x_bytes, stream, ev0, ev1);
+        case Q4_0: return launch_mfma_fmt<Q4_0>(W, p, M, (uint32_t)x_bytes, stream, ev0, ev1);
+        case Q4_K: return launch_mfma_fmt<Q4_K>(W, p, M, (uint32_t)x_bytes, stream, ev0, ev1);
+        case Q8_0: return launch_mfma_fmt<Q8_0>(W, p, M, (uint32_t)x_bytes, stream, ev0, ev1);
+        case Q6_K: return launch_mfma_fmt<Q6_K>(W, p, M, (uint32_t)x_bytes, stream, ev0, ev1);
         default: return hipErrorInvalidValue;
     }
 }

@@ -1,6 +1,5 @@
 // Small-M (2 <= M <= 32) quantized products on the matrix cores of gfx950:
-// the kernels (included by mfma.hip, fp16 activations, and mfma_f32.hip, fp32
-// activations, which are built with different code-generation options).
+// the staged and split-K kernels of fp16 activations.
 //
 // y[m][n] = sum_k W[n][k] x[m][k] is a real contraction once M > 1: each
 // weight is used M times. Here the weights are decoded to their exact
@@ -10,13 +9,7 @@
 // product is exact and the matrix core accumulates one scale block in fp32;
 // the block's scale is applied to that block's 16x16 result in fp32 (and for
 // Q4_K the minimum through a second product of x with a block of ones), so
-// the arithmetic matches the batch-1 kernels' per-block epilogue. fp32
-// activations are first scaled per (scale block, activation row) by the power
-// of two that brings the block's largest magnitude into [2^14, 2^15), then
-// split into an fp16 high and low part (x = hi + lo to 2^-22 of the value, or
-// 2^-39 of the block's largest) and multiplied as two tiles; the inverse power
-// multiplies the block's scaled result, so no value overflows fp16 or loses
-// its low bits to fp16's subnormal range.
+// the arithmetic matches the batch-1 kernels' per-block epilogue.
 //
 // Work mapping. A workgroup of W waves (four, or fewer for short matrices)
 // owns 16 W rows (16 per wave, the matrix core's N) and walks K in sub-steps of four chunks (256 weights, 128
@@ -58,34 +51,16 @@ template <> struct MfmaTraits<Q6_K> { static constexpr int SUBK = 256, NB = 16, 
 constexpr int kWeightDepth = 4; // sub-steps of weights in flight per wave
 constexpr int kUnitPad = 17;    // B-tile units per (block, k-slice): 16 rows + 1 against bank conflicts
 
-template <int FMT, int NT, bool XF32, int W>
+template <int FMT, int NT, int W>
 struct MfmaLds {
     using T = MfmaTraits<FMT>;
-    static constexpr int NTA = NT * (XF32 ? 2 : 1);           // A tiles per block (hi/lo for fp32 x)
     static constexpr int UB = T::KB == 32 ? 16 : 8;           // bytes per operand unit (8 or 4 halves)
-    static constexpr int XSC = XF32 ? T::NB * NT * 16 * 4 : 0;  // fp32 x: a power of two per (block, row)
-    static constexpr int XBUF = T::NB * NTA * 64 * UB + XSC;  // one staged activation sub-step
+    static constexpr int XBUF = T::NB * NT * 64 * UB;         // one staged activation sub-step
     static constexpr int BTILE = T::NB * 4 * kUnitPad * UB + 128;   // one wave's decoded weights (+ skew)
     static constexpr int SCALES = T::NB * 16 * 8 + 128;             // one wave's (scale, min) pairs (+ skew)
     static constexpr int WAVE = BTILE + SCALES;
     static constexpr int TOTAL = 2 * XBUF + W * WAVE;
 };
-
-// fp32 activations: the exponent k that brings a block's largest magnitude
-// `amax` into [2^14, 2^15) (fp16 holds up to 65504), 0 for a zero or
-// non-finite block, within [-126, 126] so that 2^-k is a normal fp32.
-__device__ __forceinline__ int block_shift(float amax) {
-    if (!(amax > 0.f) || !(amax <= 3.402823466e38f)) return 0;
-    const int k = 15 - __builtin_amdgcn_frexp_expf(amax);
-    return k < -126 ? -126 : (k > 126 ? 126 : k);
-}
-
-// x * 2^k split into an fp16 high part and the fp16 rounding of the rest.
-__device__ __forceinline__ void split_scaled(float x, int k, _Float16& hi, _Float16& lo) {
-    const float v = __builtin_amdgcn_ldexpf(x, k);
-    hi = (_Float16)v;
-    lo = (_Float16)(v - (float)hi);
-}
 
 // Byte offset of B-tile unit (block b, k-slice q, row n). The blocks of one
 // loader chunk are shifted by 32 bytes per chunk, so that the four loader
@@ -158,13 +133,12 @@ __device__ __forceinline__ void decode_to_tile(const ChunkData<FMT>& d0, int ln,
     }
 }
 
-template <int FMT, int NT, bool XF32, int W>
+template <int FMT, int NT, int W>
 __global__ void __launch_bounds__(64 * W) matvec_mfma(MvParams p, int M, uint32_t x_bytes) {
     using TR = MfmaTraits<FMT>;
-    using L = MfmaLds<FMT, NT, XF32, W>;
-    constexpr int SUBK = TR::SUBK, NB = TR::NB, NTA = L::NTA;
+    using L = MfmaLds<FMT, NT, W>;
+    constexpr int SUBK = TR::SUBK, NB = TR::NB;
     constexpr int XI = 16 * NT * (SUBK / 8) / (64 * W);  // activation items per thread
-    constexpr int XW = XF32 ? 2 : 1;                                // 16-byte loads per item
     extern __shared__ uint4 smem[];
     uint8_t* lds = reinterpret_cast<uint8_t*>(smem);
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -190,68 +164,29 @@ __global__ void __launch_bounds__(64 * W) matvec_mfma(MvParams p, int M, uint32_
     // Activation item of a sub-step: eight values at k8 * 8 of row mm = 16 tm
     // + m, with m fastest so that consecutive lanes write consecutive LDS units.
     constexpr int K8 = SUBK / 8;
-    auto load_x = [&](int t, uint4 (&v)[XI][XW]) {
+    auto load_x = [&](int t, uint4 (&v)[XI]) {
 #pragma unroll
         for (int i = 0; i < XI; ++i) {
             const int item = (int)threadIdx.x + 64 * W * i;
             const int mm = ((item >> 4) / K8) * 16 + (item & 15), k = t * SUBK + 8 * ((item >> 4) % K8);
             const bool ok = mm < M && k < p.K;
-            const uint32_t off = (uint32_t)(((int64_t)mm * p.ldx + k) * (XF32 ? 4 : 2));
-#pragma unroll
-            for (int h = 0; h < XW; ++h) {
-                const u32x4_t r = __builtin_amdgcn_raw_buffer_load_b128(xrs, ok ? off + 16u * h : kOobOffset, 0, 0);
-                v[i][h] = make_uint4(r.x, r.y, r.z, r.w);
-            }
+            const uint32_t off = (uint32_t)(((int64_t)mm * p.ldx + k) * 2);
+            const u32x4_t r = __builtin_amdgcn_raw_buffer_load_b128(xrs, ok ? off : kOobOffset, 0, 0);
+            v[i] = make_uint4(r.x, r.y, r.z, r.w);
         }
     };
-    auto store_x = [&](const uint4 (&v)[XI][XW], uint8_t* xb) {
+    auto store_x = [&](const uint4 (&v)[XI], uint8_t* xb) {
 #pragma unroll
         for (int i = 0; i < XI; ++i) {
             const int item = (int)threadIdx.x + 64 * W * i;
-            const int m = item & 15, k8 = (item >> 4) % K8, tm = (item >> 4) / K8;
-            uint4 parts[2];  // [0] = fp16 values (or the high parts), [1] = low parts
-            if constexpr (XF32) {
-                uint32_t hi[4], lo[4];
-                const float f[8] = {__builtin_bit_cast(float, v[i][0].x), __builtin_bit_cast(float, v[i][0].y),
-                                    __builtin_bit_cast(float, v[i][0].z), __builtin_bit_cast(float, v[i][0].w),
-                                    __builtin_bit_cast(float, v[i][1].x), __builtin_bit_cast(float, v[i][1].y),
-                                    __builtin_bit_cast(float, v[i][1].z), __builtin_bit_cast(float, v[i][1].w)};
-                // the block's largest magnitude: its items sit in lanes 16 apart
-                // (k8 = 4b + lane / 16 for 32-weight blocks, 2g + lane / 16 for 16)
-                float am = 0.f;
-#pragma unroll
-                for (int e = 0; e < 8; ++e) am = fmaxf(am, fabsf(f[e]));
-                am = fmaxf(am, __shfl_xor(am, 16));
-                if constexpr (TR::KB == 32) am = fmaxf(am, __shfl_xor(am, 32));
-                const int ks = block_shift(am);
-#pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    _Float16 h0, h1, l0, l1;
-                    split_scaled(f[2 * e], ks, h0, l0);
-                    split_scaled(f[2 * e + 1], ks, h1, l1);
-                    hi[e] = (uint32_t)__builtin_bit_cast(uint16_t, h0) | ((uint32_t)__builtin_bit_cast(uint16_t, h1) << 16);
-                    lo[e] = (uint32_t)__builtin_bit_cast(uint16_t, l0) | ((uint32_t)__builtin_bit_cast(uint16_t, l1) << 16);
-                }
-                parts[0] = make_uint4(hi[0], hi[1], hi[2], hi[3]);
-                parts[1] = make_uint4(lo[0], lo[1], lo[2], lo[3]);
-                const int blk = TR::KB == 32 ? k8 >> 2 : k8 >> 1;
-                if ((k8 & (TR::KB == 32 ? 3 : 1)) == 0)
-                    reinterpret_cast<float*>(xb + L::XBUF - L::XSC)[(blk * NT + tm) * 16 + m] =
-                        __builtin_amdgcn_ldexpf(1.0f, -ks);
+            const int m = item & 15, k8 = (item >> 4) % K8, ta = (item >> 4) / K8;
+            if constexpr (TR::KB == 32) {
+                const int b = k8 >> 2, q = k8 & 3;
+                *reinterpret_cast<uint4*>(xb + (((b * NT + ta) * 64) + q * 16 + m) * 16) = v[i];
             } else {
-                parts[0] = v[i][0];
-            }
-#pragma unroll
-            for (int h = 0; h < XW; ++h) {
-                const int ta = tm * XW + h;
-                if constexpr (TR::KB == 32) {
-                    const int b = k8 >> 2, q = k8 & 3;
-                    *reinterpret_cast<uint4*>(xb + (((b * NTA + ta) * 64) + q * 16 + m) * 16) = parts[h];
-                } else {
-                    const int g = k8 >> 1, q = 2 * (k8 & 1);
-                    *reinterpret_cast<uint2*>(xb + (((g * NTA + ta) * 64) + q * 16 + m) * 8) = make_uint2(parts[h].x, parts[h].y);
-                    *reinterpret_cast<uint2*>(xb + (((g * NTA + ta) * 64) + (q + 1) * 16 + m) * 8) = make_uint2(parts[h].z, parts[h].w);
-                }
+                const int g = k8 >> 1, q = 2 * (k8 & 1);
+                *reinterpret_cast<uint2*>(xb + (((g * NT + ta) * 64) + q * 16 + m) * 8) = make_uint2(v[i].x, v[i].y);
+                *reinterpret_cast<uint2*>(xb + (((g * NT + ta) * 64) + (q + 1) * 16 + m) * 8) = make_uint2(v[i].z, v[i].w);
             }
         }
     };
@@ -266,68 +201,28 @@ __global__ void __launch_bounds__(64 * W) matvec_mfma(MvParams p, int M, uint32_
 #pragma unroll
         for (int b = 0; b < NB; ++b) {
             const float2 s = scl[scl_index<FMT>(b, mn)];
-            if constexpr (TR::KB == 32) {
-                const h8_t B = *reinterpret_cast<const h8_t*>(bt + bt_unit<FMT>(b, mq, mn));
 #pragma unroll
-                for (int ta = 0; ta < NT; ++ta) {
-                    const f4_t z = {0.f, 0.f, 0.f, 0.f};
-                    f4_t D, D2;
-                    if constexpr (XF32) {
-                        const h8_t Ah = *reinterpret_cast<const h8_t*>(xb + ((b * NTA + 2 * ta) * 64 + lane) * 16);
-                        const h8_t Al = *reinterpret_cast<const h8_t*>(xb + ((b * NTA + 2 * ta + 1) * 64 + lane) * 16);
-                        D = __builtin_amdgcn_mfma_f32_16x16x32_f16(Al, B, __builtin_amdgcn_mfma_f32_16x16x32_f16(Ah, B, z, 0, 0, 0), 0, 0, 0);
-                        if constexpr (FMT == Q4_K) {
-                            const h8_t one = {1, 1, 1, 1, 1, 1, 1, 1};
-                            D2 = __builtin_amdgcn_mfma_f32_16x16x32_f16(Al, one, __builtin_amdgcn_mfma_f32_16x16x32_f16(Ah, one, z, 0, 0, 0), 0, 0, 0);
-                        }
-                    } else {
-                        const h8_t A = *reinterpret_cast<const h8_t*>(xb + ((b * NTA + ta) * 64 + lane) * 16);
-                        D = __builtin_amdgcn_mfma_f32_16x16x32_f16(A, B, z, 0, 0, 0);
-                        if constexpr (FMT == Q4_K) {
-                            const h8_t one = {1, 1, 1, 1, 1, 1, 1, 1};
-                            D2 = __builtin_amdgcn_mfma_f32_16x16x32_f16(A, one, z, 0, 0, 0);
-                        }
+            for (int ta = 0; ta < NT; ++ta) {
+                const f4_t z = {0.f, 0.f, 0.f, 0.f};
+                f4_t D, D2;
+                if constexpr (TR::KB == 32) {
+                    const h8_t B = *reinterpret_cast<const h8_t*>(bt + bt_unit<FMT>(b, mq, mn));
+                    const h8_t A = *reinterpret_cast<const h8_t*>(xb + ((b * NT + ta) * 64 + lane) * 16);
+                    D = __builtin_amdgcn_mfma_f32_16x16x32_f16(A, B, z, 0, 0, 0);
+                    if constexpr (FMT == Q4_K) {
+                        const h8_t one = {1, 1, 1, 1, 1, 1, 1, 1};
+                        D2 = __builtin_amdgcn_mfma_f32_16x16x32_f16(A, one, z, 0, 0, 0);
                     }
-                    if constexpr (XF32) {
-                        // the block's scaled result, times the inverse power of its activation rows
-                        const f4_t fx = *reinterpret_cast<const f4_t*>(xb + L::XBUF - L::XSC + ((b * NT + ta) * 16 + 4 * mq) * 4);
-#pragma unroll
-                        for (int j = 0; j < 4; ++j) {  // (the power of two folds exactly into the scales)
-                            float a = fmaf(s.x * fx[j], D[j], acc[ta][j]);
-                            if constexpr (FMT == Q4_K) a = fmaf(-s.y * fx[j], D2[j], a);
-                            acc[ta][j] = a;
-                        }
-                    } else {
-#pragma unroll
-                        for (int j = 0; j < 4; ++j) {
-                            float a = fmaf(s.x, D[j], acc[ta][j]);
-                            if constexpr (FMT == Q4_K) a = fmaf(-s.y, D2[j], a);
-                            acc[ta][j] = a;
-                        }
-                    }
+                } else {
+                    const h4_t B = *reinterpret_cast<const h4_t*>(bt + bt_unit<FMT>(b, mq, mn));
+                    const h4_t A = *reinterpret_cast<const h4_t*>(xb + ((b * NT + ta) * 64 + lane) * 8);
+                    D = __builtin_amdgcn_mfma_f32_16x16x16f16(A, B, z, 0, 0, 0);
                 }
-            } else {
-                const h4_t B = *reinterpret_cast<const h4_t*>(bt + bt_unit<FMT>(b, mq, mn));
 #pragma unroll
-                for (int ta = 0; ta < NT; ++ta) {
-                    const f4_t z = {0.f, 0.f, 0.f, 0.f};
-                    f4_t D;
-                    if constexpr (XF32) {
-                        const h4_t Ah = *reinterpret_cast<const h4_t*>(xb + ((b * NTA + 2 * ta) * 64 + lane) * 8);
-                        const h4_t Al = *reinterpret_cast<const h4_t*>(xb + ((b * NTA + 2 * ta + 1) * 64 + lane) * 8);
-                        D = __builtin_amdgcn_mfma_f32_16x16x16f16(Al, B, __builtin_amdgcn_mfma_f32_16x16x16f16(Ah, B, z, 0, 0, 0), 0, 0, 0);
-                    } else {
-                        const h4_t A = *reinterpret_cast<const h4_t*>(xb + ((b * NTA + ta) * 64 + lane) * 8);
-                        D = __builtin_amdgcn_mfma_f32_16x16x16f16(A, B, z, 0, 0, 0);
-                    }
-                    if constexpr (XF32) {
-                        const f4_t fx = *reinterpret_cast<const f4_t*>(xb + L::XBUF - L::XSC + ((b * NT + ta) * 16 + 4 * mq) * 4);
-#pragma unroll
-                        for (int j = 0; j < 4; ++j) acc[ta][j] = fmaf(s.x * fx[j], D[j], acc[ta][j]);
-                    } else {
-#pragma unroll
-                        for (int j = 0; j < 4; ++j) acc[ta][j] = fmaf(s.x, D[j], acc[ta][j]);
-                    }
+                for (int j = 0; j < 4; ++j) {
+                    float a = fmaf(s.x, D[j], acc[ta][j]);
+                    if constexpr (FMT == Q4_K) a = fmaf(-s.y, D2[j], a);
+                    acc[ta][j] = a;
                 }
             }
         }
@@ -338,7 +233,7 @@ __global__ void __launch_bounds__(64 * W) matvec_mfma(MvParams p, int M, uint32_
     // that enough bytes are in flight to cover HBM latency. A set is refilled
     // only after it has been decoded, never copied while its loads are pending.
     ChunkData<FMT> w[kWeightDepth];
-    uint4 xr[2][XI][XW];
+    uint4 xr[2][XI];
     load_x(0, xr[0]);
     load_x(1, xr[1]);
 #pragma unroll
@@ -514,11 +409,11 @@ __global__ void __launch_bounds__(64 * kSplitK) matvec_mfma_sk(MvParams p, int M
     }
 }
 
-template <int FMT, int NT, bool XF32, int W>
+template <int FMT, int NT, int W>
 static hipError_t launch_mfma_one(const MvParams& p, int M, uint32_t x_bytes, hipStream_t stream, hipEvent_t ev0,
                                   hipEvent_t ev1) {
-    const size_t lds = MfmaLds<FMT, NT, XF32, W>::TOTAL;
-    auto kernel = matvec_mfma<FMT, NT, XF32, W>;
+    const size_t lds = MfmaLds<FMT, NT, W>::TOTAL;
+    auto kernel = matvec_mfma<FMT, NT, W>;
     if (lds > 65536) {
         hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
                                            hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
@@ -534,19 +429,14 @@ static hipError_t launch_mfma_one(const MvParams& p, int M, uint32_t x_bytes, hi
 }
 
 // A single-wave workgroup stages all activations itself; it is kept to one
-// 16-row tile of fp16 activations, where that fits in registers.
-template <int NT, bool XF32>
-constexpr int min_waves() {
-    return NT == 1 && !XF32 ? 1 : 2;
-}
-
-template <int FMT, int NT, bool XF32>
+// 16-row tile, where that fits in registers.
+template <int FMT, int NT>
 static hipError_t launch_mfma_w(int W, const MvParams& p, int M, uint32_t x_bytes, hipStream_t stream, hipEvent_t ev0,
                                 hipEvent_t ev1) {
-    if (W == 4) return launch_mfma_one<FMT, NT, XF32, 4>(p, M, x_bytes, stream, ev0, ev1);
-    if constexpr (min_waves<NT, XF32>() == 1)
-        if (W == 1) return launch_mfma_one<FMT, NT, XF32, 1>(p, M, x_bytes, stream, ev0, ev1);
-    return launch_mfma_one<FMT, NT, XF32, 2>(p, M, x_bytes, stream, ev0, ev1);
+    if (W == 4) return launch_mfma_one<FMT, NT, 4>(p, M, x_bytes, stream, ev0, ev1);
+    if constexpr (NT == 1)
+        if (W == 1) return launch_mfma_one<FMT, NT, 1>(p, M, x_bytes, stream, ev0, ev1);
+    return launch_mfma_one<FMT, NT, 2>(p, M, x_bytes, stream, ev0, ev1);
 }
 
 }  // namespace rq

@@ -182,13 +182,28 @@ int matvec_rows(const rqmv_weight* w, int64_t first_row, int64_t rows, const voi
                         rq::k2_takes(w->fmt, rows, w->cols, m, xtype, info.cus);
     if (w->fmt != rq::F16 && m >= mfma_min && !k2_few) {
         while (done < m) {
+            if (xtype == RQMV_DTYPE_F32) {
+                // As many rows per launch as its 32-bit activation offsets reach, and
+                // 32 at least (the launch refuses them if they span 4 GiB).
+                const int64_t row = ldx * 4;
+                const int64_t reach = m > 1 ? ((int64_t)rq::kOobOffset - 1 - w->cols * 4) / row + 1 : 1;
+                const int64_t most = reach > 32 ? reach : 32;
+                const int mb = (int)(most < m - done ? most : m - done);
+                p.x = static_cast<const char*>(x) + (size_t)done * (size_t)row;
+                p.y = y + (int64_t)done * ldy;
+                const hipError_t e = rq::launch_matvec_f32(w->fmt, p, mb, info.cus, stream, done == 0 ? ev0 : nullptr,
+                                                           done + mb >= m ? ev1 : nullptr);
+                if (e != hipSuccess) return hip_fail(e, "matvec launch");
+                done += mb;
+                continue;
+            }
             const int mb = m - done > 32 ? 32 : m - done;
-            if (rq::mfma_lds_bytes(w->fmt, xtype, mb, rows, info.cus) > info.lds_limit)
+            if (rq::mfma_lds_bytes(w->fmt, mb, rows, info.cus) > info.lds_limit)
                 return fail(RQMV_EINVAL, "LDS too small");
             p.x = static_cast<const char*>(x) + (size_t)done * (size_t)ldx * esize;
             p.y = y + (int64_t)done * ldy;
             const bool first = done == 0, last = done + mb >= m;
-            hipError_t e = rq::launch_matvec_mfma(w->fmt, xtype, mb, p, info.cus, stream, first ? ev0 : nullptr,
+            hipError_t e = rq::launch_matvec_mfma(w->fmt, mb, p, info.cus, stream, first ? ev0 : nullptr,
                                                   last ? ev1 : nullptr);
             if (e != hipSuccess) return hip_fail(e, "matvec launch");
             done += mb;

@@ -1,0 +1,72 @@
+"""The matrix-core forms whose waves read fp32 activations straight from the
+caches, at the edges of their tiles: one and two row tiles per wave, the packed
+operand (up to eight rows) and one to four 16-row tiles, partial tiles, ranges
+of K with and without steps, rows whose last step or block is partial and rows
+of more than one 64-chunk group, strided rows of x and y, one value far above
+its block's others and a row of another magnitude beside it."""
+import os
+
+import numpy as np
+import pytest
+
+import oracle
+from rqmv import synth
+
+pytestmark = pytest.mark.gpu
+
+THREADS = min(16, os.cpu_count() or 1)
+FMTS = ["q8_0", "q4_0", "q4_k", "q6_k"]
+
+
+def limit(cols):
+    """Relative 2-norm of the rounding: the activations' split to 2^-22 of a
+    value, the products exact, and a chain of cols / 32 scaled block sums, each
+    a product and an addition rounded in fp32 (their errors independent:
+    2 * 2^-24 * sqrt(blocks)), with a factor of two for blocks that cancel."""
+    return 2.0 * (2.0 ** -22 + 2.0 * 2.0 ** -24 * np.sqrt(cols / 32) + 2.0 ** -23)
+
+
+def rel(a, b):
+    return float(np.linalg.norm(np.asarray(a, np.float64) - b) / np.linalg.norm(b))
+
+
+def activations(m, ldx, xdt, seed):
+    x = synth.activations_f32(m * ldx, seed=seed).reshape(m, ldx)
+    if xdt == "f16":
+        xh = synth.fp16_bits(x)
+        return xh, synth.fp16_to_f32(xh)
+    x[:, 5] *= 3e4
+    x[m - 1] *= 1e-5
+    return x, x
+
+
+def check(gpu, fmt, rows, cols, xdt, ms, pad):
+    w = synth.weights(fmt, rows, cols, seed=rows + cols)
+    W = gpu.Weight(fmt, rows, cols, w)
+    dt = gpu.DTYPE_F16 if xdt == "f16" else gpu.DTYPE_F32
+    for m in ms:
+        ldx, ldy = cols + pad, rows + pad
+        xh, x32 = activations(m, ldx, xdt, seed=m + cols)
+        yb = gpu.DeviceBuffer(4 * m * ldy)
+        yb.fill_zero()
+        W.matvec(gpu.DeviceBuffer.from_array(xh), dt, m, ldx, yb, ldy)
+        gpu.synchronize()
+        y = yb.download(np.float32).reshape(m, ldy)
+        ref = oracle.matvec_f64(fmt, w, rows, cols, x32[:, :cols], threads=THREADS)
+        for i in (range(m) if xdt == "f32" else [slice(None)]):  # (each row has a magnitude of its own)
+            assert rel(y[i, :rows] if xdt == "f32" else y[:, :rows], ref[i]) <= limit(cols), (fmt, rows, cols, m, i)
+        assert (y[:, rows:] == 0).all(), (fmt, rows, cols, m)
+    W.close()
+
+
+def shapes(fmt):
+    return [(83, 768), (300, 5376), (16, 256)] if fmt in ("q4_k", "q6_k") else [(83, 800), (300, 4160), (16, 96)]
+
+
+@pytest.mark.parametrize("fmt", FMTS)
+@pytest.mark.parametrize("rt,wk", [("1", "8"), ("2", "4"), ("2", "1")])
+def test_direct_f32(gpu, fmt, rt, wk, monkeypatch):
+    monkeypatch.setenv("RQMV_DIRECT_RT", rt)
+    monkeypatch.setenv("RQMV_DIRECT_WK", wk)
+    for n, (rows, cols) in enumerate(shapes(fmt)):
+        check(gpu, fmt, rows, cols, "f32", (5, 8, 9, 16, 17, 32, 33, 64, 77), 0 if n else 4)
