@@ -94,6 +94,12 @@ hipError_t launch_matvec_mfma(int fmt, int M, const MvParams& p, int cus, hipStr
 // activations span less than 4 GiB.
 hipError_t launch_matvec_f32(int fmt, const MvParams& p, int M, int cus, hipStream_t stream, hipEvent_t ev0 = nullptr,
                              hipEvent_t ev1 = nullptr);
+// The tiled form (mfma_tile.hip), for many activation rows. tile_takes: whether
+// a product of M rows runs in it rather than in the streaming form (fp16) or the
+// direct one (fp32).
+bool tile_takes(int fmt, int xtype, int M, int64_t rows, int64_t cols, int cus);
+hipError_t launch_matvec_tile(int fmt, int xtype, int M, const MvParams& p, int cus, hipStream_t stream,
+                              hipEvent_t ev0 = nullptr, hipEvent_t ev1 = nullptr);
 size_t mfma_lds_bytes(int fmt, int M, int64_t rows, int cus);
 
 // recipe's int(8) sum (int8.hip): Q8 activation records of `step` (32 or 256)

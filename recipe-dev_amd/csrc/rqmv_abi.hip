@@ -182,19 +182,22 @@ int matvec_rows(const rqmv_weight* w, int64_t first_row, int64_t rows, const voi
                         rq::k2_takes(w->fmt, rows, w->cols, m, xtype, info.cus);
     if (w->fmt != rq::F16 && m >= mfma_min && !k2_few) {
         while (done < m) {
-            if (xtype == RQMV_DTYPE_F32) {
-                // As many rows per launch as its 32-bit activation offsets reach, and
-                // 32 at least (the launch refuses them if they span 4 GiB).
-                const int64_t row = ldx * 4;
-                const int64_t reach = m > 1 ? ((int64_t)rq::kOobOffset - 1 - w->cols * 4) / row + 1 : 1;
-                const int64_t most = reach > 32 ? reach : 32;
-                const int mb = (int)(most < m - done ? most : m - done);
+            // The tiled form and fp32 activations run as many rows per launch as
+            // its 32-bit activation offsets reach, and 32 at least (the launch
+            // refuses them if they span 4 GiB).
+            const int64_t row = ldx * (int64_t)esize;
+            const int64_t reach = m > 1 ? ((int64_t)rq::kOobOffset - 1 - w->cols * (int64_t)esize) / row + 1 : 1;
+            const int64_t most = reach > 32 ? reach : 32;
+            const int all = (int)(most < m - done ? most : m - done);
+            const bool tile = rq::tile_takes(w->fmt, xtype, all, rows, w->cols, info.cus);
+            if (tile || xtype == RQMV_DTYPE_F32) {
                 p.x = static_cast<const char*>(x) + (size_t)done * (size_t)row;
                 p.y = y + (int64_t)done * ldy;
-                const hipError_t e = rq::launch_matvec_f32(w->fmt, p, mb, info.cus, stream, done == 0 ? ev0 : nullptr,
-                                                           done + mb >= m ? ev1 : nullptr);
+                const hipEvent_t e0 = done == 0 ? ev0 : nullptr, e1 = done + all >= m ? ev1 : nullptr;
+                const hipError_t e = tile ? rq::launch_matvec_tile(w->fmt, xtype, all, p, info.cus, stream, e0, e1)
+                                          : rq::launch_matvec_f32(w->fmt, p, all, info.cus, stream, e0, e1);
                 if (e != hipSuccess) return hip_fail(e, "matvec launch");
-                done += mb;
+                done += all;
                 continue;
             }
             const int mb = m - done > 32 ? 32 : m - done;

@@ -1,9 +1,10 @@
-"""The matrix-core forms whose waves read fp32 activations straight from the
-caches, at the edges of their tiles: one and two row tiles per wave, the packed
-operand (up to eight rows) and one to four 16-row tiles, partial tiles, ranges
-of K with and without steps, rows whose last step or block is partial and rows
-of more than one 64-chunk group, strided rows of x and y, one value far above
-its block's others and a row of another magnitude beside it."""
+"""The matrix-core forms for fp32 activations and for many activation rows, at
+the edges of their tiles: the direct form with one and two row tiles per wave,
+the packed operand (up to eight rows) and one to four 16-row tiles; the tiled
+form in each of its workgroup shapes, fp16 and fp32 activations. Partial tiles,
+ranges of K with and without steps, rows whose last step or block is partial and
+rows of more than one 64-chunk group, strided rows of x and y, one value far
+above its block's others and a row of another magnitude beside it."""
 import os
 
 import numpy as np
@@ -64,8 +65,18 @@ def shapes(fmt):
 
 
 @pytest.mark.parametrize("fmt", FMTS)
+@pytest.mark.parametrize("shape", ["11", "12", "22", "15", "14"])
+@pytest.mark.parametrize("xdt", ["f16", "f32"])
+def test_tiled(gpu, fmt, shape, xdt, monkeypatch):
+    monkeypatch.setenv("RQMV_TILE", shape)
+    for n, (rows, cols) in enumerate(shapes(fmt)):
+        check(gpu, fmt, rows, cols, xdt, (3, 16, 33, 129), 0 if n else 8)
+
+
+@pytest.mark.parametrize("fmt", FMTS)
 @pytest.mark.parametrize("rt,wk", [("1", "8"), ("2", "4"), ("2", "1")])
 def test_direct_f32(gpu, fmt, rt, wk, monkeypatch):
+    monkeypatch.setenv("RQMV_TILE", "0")
     monkeypatch.setenv("RQMV_DIRECT_RT", rt)
     monkeypatch.setenv("RQMV_DIRECT_WK", wk)
     for n, (rows, cols) in enumerate(shapes(fmt)):
