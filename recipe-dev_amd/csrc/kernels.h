@@ -59,6 +59,7 @@ struct LaunchShape {
     int block = 256;  // threads per workgroup
     int grid = 0;     // workgroups (0 = derive)
     bool k2 = false;  // two waves per row tile (matvec_int_k2)
+    int groups = 1;   // groups of activation rows along the grid's y dimension (F16 weights)
 };
 
 // Chooses G, R, block and grid for a product; honours RQMV_G / RQMV_R /

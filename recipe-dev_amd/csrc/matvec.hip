@@ -482,6 +482,10 @@ __global__ void __launch_bounds__(256) matvec_burst(MvParams p, int S) {
 template <int M, int R, bool XF32>
 __global__ void __launch_bounds__(512) matvec_f16w(MvParams p) {
     extern __shared__ uint4 smem[];
+    if constexpr (M == 16) {  // this workgroup's group of sixteen activation rows
+        p.x = static_cast<const char*>(p.x) + (int64_t)blockIdx.y * M * p.ldx * (XF32 ? 4 : 2);
+        p.y += (int64_t)blockIdx.y * M * p.ldy;
+    }
     const int nch = p.P.nch;
     const int lane = threadIdx.x & 63, g = lane & (p.G - 1), sub = lane >> p.g_shift;
     StepWalk w = make_walk(p, R, g);
@@ -713,9 +717,9 @@ static hipError_t launch_kernel(K kernel, const MvParams& p_in, const LaunchShap
         if (e != hipSuccess) return e;
     }
     if (ev0 || ev1)  // events recorded by the dispatch itself: its start and completion
-        hipExtLaunchKernelGGL(kernel, dim3(s.grid), dim3(s.block), (uint32_t)lds, stream, ev0, ev1, 0u, p);
+        hipExtLaunchKernelGGL(kernel, dim3(s.grid, s.groups), dim3(s.block), (uint32_t)lds, stream, ev0, ev1, 0u, p);
     else
-        hipLaunchKernelGGL(kernel, dim3(s.grid), dim3(s.block), lds, stream, p);
+        hipLaunchKernelGGL(kernel, dim3(s.grid, s.groups), dim3(s.block), lds, stream, p);
     return hipGetLastError();
 }
 
