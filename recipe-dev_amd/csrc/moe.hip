@@ -25,6 +25,7 @@
 namespace rq {
 
 constexpr int kMoeThreads = 256;  // workgroup size of the MoE kernels (four waves)
+constexpr int kMoeDownBatchMin = 16;  // positions from which the down product takes the batch form
 constexpr int kMoeOwnRouteMax = 2;  // positions per launch up to which every wave routes on its own
 
 static size_t al(size_t v) { return (v + 255) & ~size_t(255); }
@@ -616,6 +617,157 @@ __global__ void __launch_bounds__(BT) moe_down_kernel(MoeDims d, MoeBank down, M
     }
 }
 
+// ---- down, over a batch ----
+// The slot activations of a position are encoded once, in place (a chunk's digit
+// words and block data take 192 of its fp32 values' 256 bytes, 112 of 128 for
+// Q8_0), since every row block's workgroup of the position reads them.
+constexpr int kEncodeChunks = 64;  // chunks per workgroup
+template <int FMT>
+__global__ void __launch_bounds__(kMoeThreads) moe_encode_kernel(MoeDims d, MoeWorkspace ws, MoeBatch batch) {
+    constexpr int CW = Traits<FMT>::CW, XP = Traits<FMT>::XP, U = XP + Traits<FMT>::XR;
+    __shared__ uint4 smem[U * kEncodeChunks];
+    ws = position_ws(ws, batch.ws_stride, (int)blockIdx.y);
+    const int total = (d.top * d.hidden + d.hidden_shared) / CW, c0 = (int)blockIdx.x * kEncodeChunks;
+    const int nch = total - c0 < kEncodeChunks ? total - c0 : kEncodeChunks;
+    float* const h = ws.h + (int64_t)c0 * CW;
+    stage_all<FMT, true>(nch, nch * CW, h, 0, 1, kMoeThreads, smem, reinterpret_cast<float*>(smem + XP * nch));
+    __syncthreads();  // every value of these chunks is read
+    for (int i = (int)threadIdx.x; i < nch * U; i += kMoeThreads) {
+        const int c = i / U, u = i % U;
+        reinterpret_cast<uint4*>(h + (int64_t)c * CW)[u] = smem[u * nch + c];
+    }
+}
+
+// One position and `span` output rows (a multiple of 32) per workgroup, eight lanes
+// per row: lane g takes chunks g, g + 8, ... and keeps the NA partial sums that lanes
+// g, g + 8, ... of 8 NA lanes would (chunk g + 8 k in sum k mod NA), so that every row
+// carries the bits of the one-position form. Workgroups go to the eight XCDs in turn;
+// an XCD takes every eighth block of rows, all positions of one block before the next,
+// so that the positions that chose an expert find its rows in the XCD's L2 or close to
+// it. Bound by VALU issue: a chunk's 32 digit dots and about 60 instructions around them.
+template <int FMT>
+constexpr int down_pitch() {  // bytes of a staged chunk in LDS: lanes on consecutive chunks hit different banks
+    return (Traits<FMT>::XP + Traits<FMT>::XR) * 16 + 16;
+}
+template <int FMT, int NA>
+__global__ void __launch_bounds__(kMoeThreads) moe_down_batch_kernel(MoeDims d, MoeBank down, MoeBank down_sh,
+                                                                     MoeWorkspace ws, float* y, MoeBatch batch, int span) {
+    constexpr int CW = Traits<FMT>::CW, QP = Traits<FMT>::QP, XP = Traits<FMT>::XP, U = XP + Traits<FMT>::XR;
+    constexpr int PITCH = down_pitch<FMT>();
+    const int j8 = (int)blockIdx.x >> 3, p = j8 % batch.m, block = ((int)blockIdx.x & 7) + 8 * (j8 / batch.m);
+    if (block * span >= d.d_model) return;
+    ws = position_ws(ws, batch.ws_stride, p);
+    extern __shared__ uint4 smem[];
+    const int nch = (d.top * d.hidden + d.hidden_shared) / CW, cps = d.hidden / CW, routed_ch = d.top * cps;
+    uint8_t* const staged = reinterpret_cast<uint8_t*>(smem);
+    // per chunk: the byte offset of its first code part in its expert's first row, of its
+    // scales, its slot's weight, and the distance of its code parts (high half) and of
+    // Q6_K's d from the scales (low half)
+    uint4* const where = reinterpret_cast<uint4*>(staged + nch * PITCH);
+    for (int c = (int)threadIdx.x; c < nch; c += kMoeThreads) {
+        const bool routed = c < routed_ch;
+        const int s = routed ? c / cps : d.top, lc = routed ? c % cps : c - routed_ch;
+        const Planes& P = routed ? down.P : down_sh.P;
+        const uint32_t row0 = routed ? (uint32_t)ws.ids[s] * (uint32_t)down.rows * (uint32_t)P.row_bytes : 0u;
+        const int within = lc & 63, rest = P.nch - (lc & ~63), nb = rest > 64 ? 64 : rest;
+        const uint32_t gb = row0 + (uint32_t)(lc >> 6) * full_group_bytes<FMT>(), meta = gb + (uint32_t)(QP * nb * 16);
+        uint32_t at = meta + (uint32_t)(FMT == Q8_0 ? within * 2 : FMT == Q4_0 ? within * 4 : within / 4 * 16);
+        uint32_t dd = 0u;
+        if constexpr (FMT == Q6_K) {
+            dd = (uint32_t)((nb >> 2) * 16 + within / 4 * 2 - (within / 4 * 16 + (within & 3) * 4)) & 0xFFFFu;
+            at += (uint32_t)(within & 3) * 4u;
+        }
+        where[c] = make_uint4(gb + (uint32_t)within * 16u, at, __builtin_bit_cast(uint32_t, ws.weights[s]), (uint32_t)(nb * 16) << 16 | dd);
+    }
+    // four lanes to a chunk's 64 bytes
+    for (int i = (int)threadIdx.x; i < nch * ((U + 3) & ~3); i += kMoeThreads) {
+        const int c = (i >> 2) % nch, u = (i >> 2) / nch * 4 + (i & 3);
+        if (u < U) reinterpret_cast<uint4*>(staged + c * PITCH)[u] = reinterpret_cast<const uint4*>(ws.h + (int64_t)c * CW)[u];
+    }
+    __syncthreads();
+    const int lane = threadIdx.x & 63, g = lane & 7, wave = threadIdx.x >> 6;
+    const int n0 = block * span + wave * 8 + (lane >> 3);  // this lane's first row, then every 32nd
+    const int rounds = (nch + 7) >> 3;
+    // The rounds of all of the wave's rows in one sequence, their weights requested
+    // DEPTH - 1 rounds ahead.
+    int fk = 0, fn = n0;  // the next round to request
+    auto fetch = [&](ChunkData<FMT>& cd, float& w) {
+        int c = 8 * fk + g;
+        c = c < nch ? c : nch - 1;
+        const uint4 at = where[c];
+        w = __builtin_bit_cast(float, at.z);
+        const bool routed = c < routed_ch;
+        const uint8_t* const base = routed ? down.P.base : down_sh.P.base;
+        const uint32_t row = (uint32_t)(fn < d.d_model ? fn : d.d_model - 1) * (uint32_t)(routed ? down.P.row_bytes : down_sh.P.row_bytes);
+#pragma unroll
+        for (int h = 0; h < QP; ++h) cd.q[h] = ld16(base + (row + at.x + (uint32_t)h * (at.w >> 16)));
+        const uint8_t* const mt = base + (row + at.y);
+        if constexpr (FMT == Q4_K) cd.meta = ld16(mt);
+        else if constexpr (FMT == Q6_K)
+            cd.meta = make_uint4(*reinterpret_cast<const uint32_t*>(mt),
+                                 *reinterpret_cast<const uint16_t*>(base + (row + at.y + (uint32_t)(int)(int16_t)(at.w & 0xFFFFu))), 0, 0);
+        else if constexpr (FMT == Q4_0) cd.meta = make_uint4(*reinterpret_cast<const uint32_t*>(mt), 0, 0, 0);
+        else cd.meta = make_uint4(*reinterpret_cast<const uint16_t*>(mt), 0, 0, 0);
+        if (++fk == rounds) {
+            fk = 0;
+            fn += 32;
+        }
+    };
+    float acc[NA];
+#pragma unroll
+    for (int a = 0; a < NA; ++a) acc[a] = 0.f;
+    int k = 0, n = n0;
+    auto round = [&](const ChunkData<FMT>& cd, float w) {
+        const int c = 8 * k + g;
+        float sum = acc[0];
+        if (c < nch) {
+            // (Q4_K's scale fields go by the chunk's place in its superblock, which the
+            // slots' whole superblocks leave the same)
+            const uint4* const x = reinterpret_cast<const uint4*>(staged + c * PITCH);
+            uint4 xv[XP];
+            uint4 bv[2];
+#pragma unroll
+            for (int j = 0; j < XP; ++j) xv[j] = x[j];
+            bv[0] = x[XP];
+            bv[1] = x[XP + 1];
+            float part = 0.f;
+            dot_int<FMT>(cd, c, xv, bv, part);
+            if (__builtin_expect(wave_has_outlier(bv[0]), 0)) dot_outliers<FMT>(cd, c, x + XP, 1, part);
+            sum = fmaf(w, part, sum);
+        }
+        // the sums rotate: round k's stands in acc[0]
+#pragma unroll
+        for (int a = 0; a + 1 < NA; ++a) acc[a] = acc[a + 1];
+        acc[NA - 1] = sum;
+        if (++k < rounds) return;
+        // sum a stands in acc[(a - rounds) mod NA]; the tree over lanes g, g + 8, ..
+        float t[NA];
+#pragma unroll
+        for (int a = 0; a < NA; ++a) t[a] = group_sum(acc[a], 8);
+        float v = t[0];
+        if constexpr (NA == 2) v = t[0] + t[1];
+        if constexpr (NA == 4) v = rounds & 1 ? (t[3] + t[0]) + (t[1] + t[2]) : (t[0] + t[1]) + (t[2] + t[3]);
+        if (g == 7 && n < d.d_model) y[batch.y_stride * p + n] = v;
+#pragma unroll
+        for (int a = 0; a < NA; ++a) acc[a] = 0.f;
+        k = 0;
+        n += 32;
+    };
+    constexpr int DEPTH = 4;
+    const int total = rounds * (span / 32);
+    ChunkData<FMT> cd[DEPTH];
+    float w[DEPTH];
+#pragma unroll
+    for (int i = 0; i < DEPTH - 1; ++i) fetch(cd[i], w[i]);
+    for (int t0 = 0; t0 < total; t0 += DEPTH)
+#pragma unroll
+        for (int i = 0; i < DEPTH; ++i) {
+            if (t0 + i >= total) break;
+            fetch(cd[(i + DEPTH - 1) % DEPTH], w[(i + DEPTH - 1) % DEPTH]);
+            round(cd[i], w[i]);
+        }
+}
+
 static int lanes_for(int64_t nch) {
     int G = 64;
     while (G > 8 && G > nch) G >>= 1;
@@ -732,6 +884,29 @@ static hipError_t down_fmt(const MoeDims& d, const MoeBank& down, const MoeBank&
     // / 50.6 / 79.0 / 135.3). RQMV_MOE_DOWN_WIDE=0/1 and RQMV_MOE_DOWN_THREADS
     // override the workgroup size, RQMV_MOE_DOWN_SPLIT=0/1 the split form (one
     // or two positions, 32 lanes).
+    // Batches of 16 positions or more: the slot activations encoded once, then 64 or
+    // 128 rows of one position per workgroup, XCD by XCD (moe_down_batch_kernel). On the
+    // gguf_moe workload, us per step at 8 / 16 / 64 / 512 positions: 48.8 / 75.9 / 193.5 /
+    // 1422 in the form below against 49.5 / 67.4 / 159.0 / 1027 (64, 64, 128, 128 rows;
+    // 32 rows 51.0 / 68.8 / 171.5 / 1105). Its weights are read with ordinary loads: with
+    // the non-temporal ones of the one-position form, which mark lines for early
+    // eviction, the same steps took 50 / 74.6 / 174.8 / 1223.
+    const size_t blds = (size_t)nch * (size_t)(down_pitch<FMT>() + 16);
+    if (G <= 32 && blds <= 65536 && env_flag("RQMV_MOE_DOWN_BATCH", b.m >= kMoeDownBatchMin)) {
+        const char* senv = getenv("RQMV_MOE_DOWN_SPAN");
+        const int span = senv && *senv ? atoi(senv) / 32 * 32 : b.m >= 48 ? 128 : 64;
+        if (span < 32) return hipErrorInvalidValue;
+        hipLaunchKernelGGL(moe_encode_kernel<FMT>, dim3((nch + kEncodeChunks - 1) / kEncodeChunks, b.m), dim3(kMoeThreads),
+                           0, stream, d, ws, b);
+        hipError_t e = hipGetLastError();
+        if (e != hipSuccess) return e;
+        const int blocks = (d.d_model + span - 1) / span;
+        const int64_t wgs = (int64_t)((blocks + 7) / 8 * 8) * b.m;
+        if (wgs > 0x7FFFFFFF) return hipErrorInvalidValue;
+        auto kernel = G == 32 ? moe_down_batch_kernel<FMT, 4> : G == 16 ? moe_down_batch_kernel<FMT, 2> : moe_down_batch_kernel<FMT, 1>;
+        hipLaunchKernelGGL(kernel, dim3((unsigned)wgs), dim3(kMoeThreads), blds, stream, d, down, down_sh, ws, y, b, span);
+        return hipGetLastError();
+    }
     int threads = env_flag("RQMV_MOE_DOWN_WIDE", b.m >= 2) ? (b.m >= 3 ? 1024 : 512) : kMoeThreads;
     const char* tenv = getenv("RQMV_MOE_DOWN_THREADS");
     if (tenv && *tenv) {
