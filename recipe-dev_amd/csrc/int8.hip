@@ -31,6 +31,8 @@
 #include <hip/hip_runtime.h>
 
 #include "chunk.h"
+#include <stdlib.h>
+
 #include "kernels.h"
 
 namespace rq {
@@ -420,6 +422,89 @@ __global__ __launch_bounds__(kI8Threads) void int8_slices_kernel(I8Launch p) {
     if ((lane & 31) == 0 && (mine == 0 || two)) p.y[(int64_t)blockIdx.y * p.ldy + row0 + mine] = acc;
 }
 
+// Batches of Q8_0 products: MR activation rows per workgroup, whose records stand in
+// LDS side by side; each wave reads its two weight rows once for all of them. Every
+// output sees the operations of the one-row kernel in their order. Q8_0 5120x5120 at
+// 4 / 8 / 15 rows, step 32: 16.8 / 30.1 / 53.1 us with a workgroup per activation row
+// -> 14.7 (two rows) / 22.3 (four) / 34.7 (four; two 39.2); four rows by fours 18.1.
+// Bound by the records' LDS reads and the sums' round trip. The other formats, whose
+// chunks take twice the LDS traffic for their bytes, are no faster or slower (Q4_K
+// 4096->14336 at 4 / 8 rows 29.8 / 55.1 -> 28.6 / 49.2 by fours, 2390 rows of 1792
+// 7.3 / 10.5 -> 10.5 / 12.4) and keep a workgroup per activation row.
+__host__ __device__ inline int i8_row_bytes(int K) {  // codes, steps and inverses of one activation row
+    const int tail = (K >> 5) + ((K + 255) >> 8);
+    return K + ((tail + 3) & ~3) * 4;
+}
+template <int MR>
+__device__ __forceinline__ float* stage_record_rows(const I8Launch& p, int step, uint8_t* lds) {
+    const int stride = i8_row_bytes(p.K), m0 = (int)blockIdx.y * MR;
+    for (int r = 0; r < MR; ++r) {
+        const int m = m0 + r < p.M ? m0 + r : p.M - 1;
+        float* const xd = reinterpret_cast<float*>(lds + r * stride + p.K);
+        q8_records(p.x + (int64_t)m * p.ldx, p.K, step, xd, reinterpret_cast<int8_t*>(lds + r * stride), xd + (p.K >> 5),
+                   (int)threadIdx.x, kI8Threads);
+    }
+    return reinterpret_cast<float*>(lds + MR * stride) + ((int)threadIdx.x >> 6) * 512;
+}
+
+template <int FMT, int MR>
+__global__ __launch_bounds__(kI8Threads) void int8_slices_rows_kernel(I8Launch p) {
+    constexpr int CS = chunk_slices<FMT>();
+    extern __shared__ __align__(16) uint8_t i8_lds[];
+    float* const rowbuf = stage_record_rows<MR>(p, p.step, i8_lds);
+    const int stride = i8_row_bytes(p.K), wave = (int)threadIdx.x >> 6, lane = (int)threadIdx.x & 63;
+    const int64_t row0 = (int64_t)blockIdx.x * kI8Rows + 2 * wave;
+    if (row0 >= p.rows) return;
+    const bool two = row0 + 1 < p.rows;
+    const int slices = p.K >> 4, nch = p.P.nch, mine = lane >> 5, l = lane & 31;
+    float acc[MR];
+#pragma unroll
+    for (int r = 0; r < MR; ++r) acc[r] = 0.f;
+    for (int c0 = 0; c0 < nch; c0 += 64) {
+        const int c = c0 + lane;
+        ChunkData<FMT> A, B;
+        if (c < nch) {
+            load_chunk<FMT>(p.P, row0, c, A);
+            if (two) load_chunk<FMT>(p.P, row0 + 1, c, B);
+        }
+        const int base = c0 * CS;  // first slice of the pass
+        const float* mybuf = rowbuf + 256 * mine;
+#pragma unroll
+        for (int r = 0; r < MR; ++r) {
+            if (c < nch) {
+                const int8_t* xc = reinterpret_cast<const int8_t*>(i8_lds + r * stride);
+                const float* xd = reinterpret_cast<const float*>(i8_lds + r * stride + p.K);
+                float va[CS], vb[CS] = {};
+                chunk_values<FMT>(A, c, xc, xd, va);
+                if (two) chunk_values<FMT>(B, c, xc, xd, vb);
+#pragma unroll
+                for (int t = 0; t < CS; ++t) {
+                    rowbuf[lane * CS + t] = va[t];
+                    rowbuf[256 + lane * CS + t] = vb[t];
+                }
+            }
+            __builtin_amdgcn_wave_barrier();
+#pragma unroll
+            for (int j = 0; j < 2 * CS; ++j) {
+                const int s = base + l + 32 * j;
+                if (s < slices) acc[r] = acc[r] + mybuf[l + 32 * j];
+            }
+            __builtin_amdgcn_wave_barrier();
+        }
+    }
+#pragma unroll
+    for (int r = 0; r < MR; ++r) {
+        float v = acc[r];
+        v = v + lane_xor<16>(v);
+        v = v + lane_xor<8>(v);
+        v = v + lane_xor<4>(v);
+        v = v + lane_xor<2>(v);
+        v = v + lane_xor<1>(v);
+        const int m = (int)blockIdx.y * MR + r;
+        if (l == 0 && (mine == 0 || two) && m < p.M) p.y[(int64_t)m * p.ldy + row0 + mine] = v;
+    }
+}
+
 // Q4_K at a 256 step (amd-nv-cpu.ll:1545-1733). Lane i decodes chunk i of a
 // pass: quarter i%4 of block i/4, whose two sub-blocks give the quarter's
 // exact ints (scale times dot, minimum times code sum). Each pass leaves, per
@@ -595,27 +680,53 @@ size_t int8_lds_bytes(int64_t cols) {
     return (size_t)cols + ((tail + 3) & ~size_t(3)) * 4 + (size_t)(kI8Threads / 64) * 2048;
 }
 
+// Activation rows per workgroup of a Q8_0 batch: four from eight rows, two from four,
+// where their records fit 64 KiB of LDS. RQMV_I8_ROWS=1/2/4 overrides it for tuning.
+static int int8_rows(int M, int K) {
+    const char* env = getenv("RQMV_I8_ROWS");
+    const int want = env && *env ? atoi(env) : M >= 8 ? 4 : M >= 4 ? 2 : 1;
+    int mr = want >= 4 ? 4 : want >= 2 ? 2 : 1;
+    while (mr > 1 && (size_t)mr * i8_row_bytes(K) + (size_t)(kI8Threads / 64) * 2048 > 65536) mr >>= 1;
+    return mr;
+}
+
+template <int FMT>
+static hipError_t launch_slices(const I8Launch& p, hipStream_t stream) {
+    const int mr = FMT == Q8_0 ? int8_rows(p.M, p.K) : 1;
+    const dim3 grid((unsigned)((p.rows + kI8Rows - 1) / kI8Rows), (unsigned)((p.M + mr - 1) / mr));
+    size_t lds = int8_lds_bytes(p.K);
+    auto kernel = int8_slices_kernel<FMT>;
+    if constexpr (FMT == Q8_0) {
+        if (mr > 1) {
+            lds = (size_t)mr * i8_row_bytes(p.K) + (size_t)(kI8Threads / 64) * 2048;
+            kernel = mr == 4 ? int8_slices_rows_kernel<FMT, 4> : int8_slices_rows_kernel<FMT, 2>;
+        }
+    }
+    hipLaunchKernelGGL(kernel, grid, dim3(kI8Threads), lds, stream, p);
+    return hipGetLastError();
+}
+
 hipError_t launch_matvec_int8(int fmt, const Planes& P, int64_t rows, int K, const float* x, int M, int64_t ldx,
                               float* y, int64_t ldy, int step, int tail, hipStream_t stream) {
     I8Launch p{P, rows, K, x, ldx, y, ldy, M, step, tail};
     const dim3 grid((unsigned)((rows + kI8Rows - 1) / kI8Rows), (unsigned)M);
     const size_t lds = int8_lds_bytes(K);
     const bool blocks256 = step == 256 && (fmt == Q4_K || fmt == Q6_K);
-    if (blocks256 && fmt == Q4_K)
+    if (blocks256 && fmt == Q4_K) {
         hipLaunchKernelGGL(int8_q4k256_kernel, grid, dim3(kI8Threads), lds, stream, p);
-    else if (blocks256)
+        return hipGetLastError();
+    }
+    if (blocks256) {
         hipLaunchKernelGGL(int8_q6k256_kernel, grid, dim3(kI8Threads), lds, stream, p);
-    else if (fmt == Q4_K)
-        hipLaunchKernelGGL(int8_slices_kernel<Q4_K>, grid, dim3(kI8Threads), lds, stream, p);
-    else if (fmt == Q6_K)
-        hipLaunchKernelGGL(int8_slices_kernel<Q6_K>, grid, dim3(kI8Threads), lds, stream, p);
-    else if (fmt == Q8_0)
-        hipLaunchKernelGGL(int8_slices_kernel<Q8_0>, grid, dim3(kI8Threads), lds, stream, p);
-    else if (fmt == Q4_0)
-        hipLaunchKernelGGL(int8_slices_kernel<Q4_0>, grid, dim3(kI8Threads), lds, stream, p);
-    else
-        return hipErrorInvalidValue;
-    return hipGetLastError();
+        return hipGetLastError();
+    }
+    switch (fmt) {
+        case Q4_K: return launch_slices<Q4_K>(p, stream);
+        case Q6_K: return launch_slices<Q6_K>(p, stream);
+        case Q8_0: return launch_slices<Q8_0>(p, stream);
+        case Q4_0: return launch_slices<Q4_0>(p, stream);
+        default: return hipErrorInvalidValue;
+    }
 }
 
 hipError_t launch_q8_records(const float* x, int K, int step, float* d, int8_t* codes, hipStream_t stream) {

@@ -157,3 +157,18 @@ def test_int8_profile_storage(gpu, fmt, step):
     x = np.stack([synth.activations_f32(cols, seed=20 + i) for i in range(2)])
     assert _bits_equal(gpu.contract_int8(W, x, step), oracle.int8_matvec(sfmt, stored, rows, cols, x, step))
     assert np.array_equal(W.unpack(), stored)
+
+
+@pytest.mark.parametrize("step", [32, 256])
+@pytest.mark.parametrize("mr", ["1", "2", "4"])
+def test_q8_0_batches_by_rows_per_workgroup(gpu, mr, step, monkeypatch):
+    """Q8_0 batches with one, two and four activation rows per workgroup: whole and
+    partial groups, one row of a pair, a partial last pass and a partial last step."""
+    monkeypatch.setenv("RQMV_I8_ROWS", mr)
+    for rows, cols, m in ((35, 96, 3), (16, 2112, 7), (1, 4096, 9)):
+        w = synth.weights("q8_0", rows, cols, seed=rows)
+        x = np.stack([synth.activations_f32(cols, seed=50 + i) for i in range(m)])
+        W = gpu.Weight("q8_0", rows, cols, w)
+        got = gpu.contract_int8(W, x, step)
+        want = oracle.int8_matvec("q8_0", w, rows, cols, x, step)
+        assert np.array_equal(np.asarray(got, np.float32).view(np.uint32), np.asarray(want, np.float32).view(np.uint32))
