@@ -68,8 +68,12 @@ __device__ __forceinline__ void load_record(const float* __restrict__ xr, float4
     for (int q = 0; q < 8; ++q) xv[q] = reinterpret_cast<const float4*>(xr)[q];
 }
 
-// The 32 codes of a record in registers: clamp(round-half-even(x * inverse),
-// -128, 127) (amd-nv-cpu.ll:1484-1490), written to LDS.
+// A code: clamp(round-half-even(x * inverse), -128, 127) (amd-nv-cpu.ll:1484-1490).
+__device__ __forceinline__ int record_code(float x, float inverse) {
+    return (int)fminf(fmaxf(__builtin_rintf(x * inverse), -128.f), 127.f);
+}
+
+// The 32 codes of a record in registers, written to LDS.
 __device__ __forceinline__ void record_codes(const float4 (&xv)[8], float inverse, int8_t* out) {
     uint32_t w[8];
 #pragma unroll
@@ -77,10 +81,7 @@ __device__ __forceinline__ void record_codes(const float4 (&xv)[8], float invers
         const float f[4] = {xv[q].x, xv[q].y, xv[q].z, xv[q].w};
         uint32_t word = 0;
 #pragma unroll
-        for (int k = 0; k < 4; ++k) {
-            const float rr = __builtin_rintf(f[k] * inverse);
-            word |= ((uint32_t)(int)fminf(fmaxf(rr, -128.f), 127.f) & 0xffu) << (8 * k);
-        }
+        for (int k = 0; k < 4; ++k) word |= ((uint32_t)record_code(f[k], inverse) & 0xffu) << (8 * k);
         w[q] = word;
     }
     reinterpret_cast<uint4*>(out)[0] = make_uint4(w[0], w[1], w[2], w[3]);
@@ -104,54 +105,107 @@ __device__ __forceinline__ void record_from_registers(const float4 (&xv)[8], flo
     d[r] = dd;
 }
 
-// The Q8 records of one activation row of K inputs (16-byte aligned) into
-// LDS: codes[K], d[K/32], and ginv[ceil(K/256)] scratch for a 256 step.
-// Step 32: one thread per record scans its 32 inputs. Step 256: recipe's lane
-// v keeps the first largest magnitude among input v of the step's 32-value
-// blocks (amd-nv-cpu.ll:1408-1440), computed here by one thread per (step,
-// lane) into `codes` (free until the codes are written); one thread per step
-// then takes the extreme over its 32 lanes. Ends with a barrier.
-__device__ __forceinline__ void q8_records(const float* __restrict__ x, int K, int step, float* d, int8_t* codes,
-                                           float* ginv, int tid, int nthreads) {
-    const int blocks = K >> 5;
+// The value of lane ^ OFF (OFF < 32, within the lane's 32-lane half), through
+// DPP and the 16-lane swap rather than the LDS crossbar: quad permutations
+// for 1 and 2, row shifts by 4 either way for 4, a row rotation by 8 for 8,
+// v_permlane16_swap for 16. Each lane then adds exactly the partner
+// __shfl_xor would give it, so the butterflies keep their bits.
+template <int OFF>
+__device__ __forceinline__ float lane_xor(float v) {
+    const int iv = __builtin_bit_cast(int, v);
+    if constexpr (OFF == 1) return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, iv, 0xB1, 0xf, 0xf, false));
+    if constexpr (OFF == 2) return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, iv, 0x4E, 0xf, 0xf, false));
+    if constexpr (OFF == 4) {
+        const int up = __builtin_amdgcn_update_dpp(0, iv, 0x114, 0xf, 0xf, false);    // row_shr:4 (lane - 4)
+        const int down = __builtin_amdgcn_update_dpp(0, iv, 0x104, 0xf, 0xf, false);  // row_shl:4 (lane + 4)
+        return __builtin_bit_cast(float, (threadIdx.x & 4) ? up : down);
+    }
+    if constexpr (OFF == 8) return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, iv, 0x128, 0xf, 0xf, false));
+    if constexpr (OFF == 16) {
+        float a = v, b = v;
+        asm volatile("s_nop 1\n\tv_permlane16_swap_b32 %0, %1" : "+v"(a), "+v"(b));
+        return (threadIdx.x & 16) ? a : b;
+    }
+    static_assert(OFF == 1 || OFF == 2 || OFF == 4 || OFF == 8 || OFF == 16, "lane_xor: 1, 2, 4, 8 or 16");
+    return v;
+}
+
+// LDS of one activation row's records: codes[K], d[K/32] and spare words.
+__host__ __device__ inline int i8_row_bytes(int K) {
+    const int tail = (K >> 5) + ((K + 255) >> 8);
+    return K + ((tail + 3) & ~3) * 4;
+}
+
+// The Q8 records of MR activation rows (16-byte aligned) from row m0 on, the last of
+// the M rows again past it, into LDS, row r at r * i8_row_bytes(K). All rows' records
+// are spread over the workgroup at once. Ends with a barrier.
+// Step 32: one thread per record scans its 32 inputs. Step 256: recipe's lane v keeps
+// the first largest magnitude among input v of the step's 32-value blocks
+// (amd-nv-cpu.ll:1408-1440): 32 lanes per step each hold those inputs, take the extreme
+// over the lanes by exchanges and code what they hold. With one thread per (step, lane), then one per
+// step over 32 LDS reads, then one per record, a row's records took about 3 us of a
+// workgroup: Q4_K 1111x2048, one and two rows 6.6 -> 5.3 us, Q6_K 14336 x 4096 at
+// eight rows, a workgroup a row, 78 -> 70.
+template <int MR>
+__device__ __forceinline__ void q8_record_rows(const float* __restrict__ x, int64_t ldx, int m0, int M, int K, int step,
+                                               uint8_t* lds, int tid) {
+    const int blocks = K >> 5, stride = i8_row_bytes(K);
+    auto row_of = [&](int r) { return x + (int64_t)(m0 + r < M ? m0 + r : M - 1) * ldx; };
     if (step == 32) {
-        for (int r = tid; r < blocks; r += nthreads) {
+        for (int i = tid; i < MR * blocks; i += kI8Threads) {
+            const int r = MR == 1 ? 0 : i / blocks, b = i - r * blocks;
             float4 xv[8];
-            load_record(x + r * 32, xv);
-            record_from_registers(xv, d, codes, r);
+            load_record(row_of(r) + b * 32, xv);
+            record_from_registers(xv, reinterpret_cast<float*>(lds + r * stride + K), reinterpret_cast<int8_t*>(lds + r * stride), b);
         }
         __syncthreads();
         return;
     }
-    const int groups = (blocks + 7) >> 3;
-    float* lane_best = reinterpret_cast<float*>(codes);  // groups * 32 floats <= K bytes
-    for (int i = tid; i < groups * 32; i += nthreads) {
-        const int g = i >> 5, v = i & 31;
-        const int b1 = min(g * 8 + 8, blocks);
-        float e = 0.f;
-        for (int b = g * 8; b < b1; ++b) {
-            const float xv = x[b * 32 + v];
-            if (fabsf(xv) > fabsf(e)) e = xv;
+    constexpr int U = 4, HALVES = kI8Threads / 32;  // steps a half-wave loads at once; half-waves
+    const int groups = (blocks + 7) >> 3, items = MR * groups, v = tid & 31;
+    const bool whole = (blocks & 7) == 0;
+    for (int i0 = tid >> 6 << 1; i0 < items; i0 += U * HALVES) {  // (wave-uniform: the exchanges need every lane)
+        float xv[U][8];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            if (i0 + u * HALVES >= items) break;
+            const int i = min(i0 + u * HALVES + ((tid >> 5) & 1), items - 1), r = MR == 1 ? 0 : i / groups, g = i - r * groups;
+            const float* const at = row_of(r) + g * 256 + v;
+            if (whole) {
+#pragma unroll
+                for (int b = 0; b < 8; ++b) xv[u][b] = at[b * 32];
+            } else {
+#pragma unroll
+                for (int b = 0; b < 8; ++b) xv[u][b] = g * 8 + b < blocks ? at[b * 32] : 0.f;
+            }
         }
-        lane_best[i] = e;
-    }
-    __syncthreads();
-    for (int g = tid; g < groups; g += nthreads) {
-        float e = 0.f;
-        for (int v = 0; v < 32; ++v) {
-            const float p = lane_best[g * 32 + v];
-            if (extreme_wins(p, e)) e = p;
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            if (i0 + u * HALVES >= items) break;
+            const int i = i0 + u * HALVES + ((tid >> 5) & 1), r = MR == 1 ? 0 : i / groups, g = i - r * groups;
+            float e = 0.f;
+#pragma unroll
+            for (int b = 0; b < 8; ++b)  // (zeros past the row's end never win)
+                if (fabsf(xv[u][b]) > fabsf(e)) e = xv[u][b];
+            float o = lane_xor<16>(e);
+            if (extreme_wins(o, e)) e = o;
+            o = lane_xor<8>(e);
+            if (extreme_wins(o, e)) e = o;
+            o = lane_xor<4>(e);
+            if (extreme_wins(o, e)) e = o;
+            o = lane_xor<2>(e);
+            if (extreme_wins(o, e)) e = o;
+            o = lane_xor<1>(e);
+            if (extreme_wins(o, e)) e = o;
+            float inverse, dd;
+            step_of(e, inverse, dd);
+            if (i >= items) continue;
+            int8_t* const codes = reinterpret_cast<int8_t*>(lds + r * stride) + g * 256 + v;
+#pragma unroll
+            for (int b = 0; b < 8; ++b)
+                if (whole || g * 8 + b < blocks) codes[b * 32] = (int8_t)record_code(xv[u][b], inverse);
+            if (v < 8 && g * 8 + v < blocks) reinterpret_cast<float*>(lds + r * stride + K)[g * 8 + v] = dd;
         }
-        float inverse, dd;
-        step_of(e, inverse, dd);
-        ginv[g] = inverse;
-        for (int b = g * 8; b < min(g * 8 + 8, blocks); ++b) d[b] = dd;
-    }
-    __syncthreads();
-    for (int r = tid; r < blocks; r += nthreads) {
-        float4 xv[8];
-        load_record(x + r * 32, xv);
-        record_codes(xv, ginv[r >> 3], codes + r * 32);
     }
     __syncthreads();
 }
@@ -296,15 +350,15 @@ struct I8Launch {
     int tail;
 };
 
-// LDS: the records' codes (K bytes), steps (K/32 floats) and per-step
-// inverses (ceil(K/256) floats), then per wave two rows of 256 slice values.
+// LDS: the records' codes (K bytes), steps (K/32 floats) and ceil(K/256) spare
+// words, then per wave two rows of 256 slice values.
 __device__ __forceinline__ void stage_records(const I8Launch& p, int step, int8_t*& xc, float*& xd, float*& rowbuf) {
     extern __shared__ __align__(16) uint8_t i8_lds[];
     xc = reinterpret_cast<int8_t*>(i8_lds);
     xd = reinterpret_cast<float*>(i8_lds + p.K);
     const int tail_floats = (p.K >> 5) + ((p.K + 255) >> 8);
     rowbuf = xd + ((tail_floats + 3) & ~3) + ((int)threadIdx.x >> 6) * 512;
-    q8_records(p.x + (int64_t)blockIdx.y * p.ldx, p.K, step, xd, xc, xd + (p.K >> 5), (int)threadIdx.x, kI8Threads);
+    q8_record_rows<1>(p.x, p.ldx, (int)blockIdx.y, p.M, p.K, step, i8_lds, (int)threadIdx.x);
 }
 
 // Exact int sums over the four lanes of a quad (one 256-value block).
@@ -313,31 +367,6 @@ __device__ __forceinline__ int quad_sum(int v) {
     return v + __builtin_amdgcn_update_dpp(0, v, 0x4E, 0xf, 0xf, false);  // lane ^ 2
 }
 __device__ __forceinline__ int lane_int(int v, int lane) { return __builtin_amdgcn_readlane(v, lane); }
-// The value of lane ^ OFF (OFF < 32, within the lane's 32-lane half), through
-// DPP and the 16-lane swap rather than the LDS crossbar: quad permutations
-// for 1 and 2, row shifts by 4 either way for 4, a row rotation by 8 for 8,
-// v_permlane16_swap for 16. Each lane then adds exactly the partner
-// __shfl_xor would give it, so the butterflies keep their bits.
-template <int OFF>
-__device__ __forceinline__ float lane_xor(float v) {
-    const int iv = __builtin_bit_cast(int, v);
-    if constexpr (OFF == 1) return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, iv, 0xB1, 0xf, 0xf, false));
-    if constexpr (OFF == 2) return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, iv, 0x4E, 0xf, 0xf, false));
-    if constexpr (OFF == 4) {
-        const int up = __builtin_amdgcn_update_dpp(0, iv, 0x114, 0xf, 0xf, false);    // row_shr:4 (lane - 4)
-        const int down = __builtin_amdgcn_update_dpp(0, iv, 0x104, 0xf, 0xf, false);  // row_shl:4 (lane + 4)
-        return __builtin_bit_cast(float, (threadIdx.x & 4) ? up : down);
-    }
-    if constexpr (OFF == 8) return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, iv, 0x128, 0xf, 0xf, false));
-    if constexpr (OFF == 16) {
-        float a = v, b = v;
-        asm volatile("s_nop 1\n\tv_permlane16_swap_b32 %0, %1" : "+v"(a), "+v"(b));
-        return (threadIdx.x & 16) ? a : b;
-    }
-    static_assert(OFF == 1 || OFF == 2 || OFF == 4 || OFF == 8 || OFF == 16, "lane_xor: 1, 2, 4, 8 or 16");
-    return v;
-}
-
 __device__ __forceinline__ float lane_float(float v, int lane) {
     return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), lane));
 }
@@ -422,29 +451,17 @@ __global__ __launch_bounds__(kI8Threads) void int8_slices_kernel(I8Launch p) {
     if ((lane & 31) == 0 && (mine == 0 || two)) p.y[(int64_t)blockIdx.y * p.ldy + row0 + mine] = acc;
 }
 
-// Batches of Q8_0 products: MR activation rows per workgroup, whose records stand in
-// LDS side by side; each wave reads its two weight rows once for all of them. Every
-// output sees the operations of the one-row kernel in their order. Q8_0 5120x5120 at
-// 4 / 8 / 15 rows, step 32: 16.8 / 30.1 / 53.1 us with a workgroup per activation row
-// -> 14.7 (two rows) / 22.3 (four) / 34.7 (four; two 39.2); four rows by fours 18.1.
-// Bound by the records' LDS reads and the sums' round trip. The other formats, whose
-// chunks take twice the LDS traffic for their bytes, are no faster or slower (Q4_K
-// 4096->14336 at 4 / 8 rows 29.8 / 55.1 -> 28.6 / 49.2 by fours, 2390 rows of 1792
-// 7.3 / 10.5 -> 10.5 / 12.4) and keep a workgroup per activation row.
-__host__ __device__ inline int i8_row_bytes(int K) {  // codes, steps and inverses of one activation row
-    const int tail = (K >> 5) + ((K + 255) >> 8);
-    return K + ((tail + 3) & ~3) * 4;
-}
+// Batches: MR activation rows per workgroup, whose records stand in LDS side by side;
+// each wave reads and unpacks its two weight rows once for all of them. Every output sees
+// the operations of the one-row kernel in their order. Step 32, us at 4 / 8 rows with a
+// workgroup per activation row -> four rows a workgroup: Q4_K 4096->14336 27.7 / 52.5 ->
+// 22.9 / 37.8, Q6_K 33.5 / 62.0 -> 22.6 / 35.9, Q4_0 33.2 / 61.6 -> 24.4 / 35.5; Q8_0
+// 5120x5120 14.3 / 25.9 -> 13.1 (two rows) / 20.5. Bound by the records' LDS reads and
+// the sums' round trip.
 template <int MR>
 __device__ __forceinline__ float* stage_record_rows(const I8Launch& p, int step, uint8_t* lds) {
-    const int stride = i8_row_bytes(p.K), m0 = (int)blockIdx.y * MR;
-    for (int r = 0; r < MR; ++r) {
-        const int m = m0 + r < p.M ? m0 + r : p.M - 1;
-        float* const xd = reinterpret_cast<float*>(lds + r * stride + p.K);
-        q8_records(p.x + (int64_t)m * p.ldx, p.K, step, xd, reinterpret_cast<int8_t*>(lds + r * stride), xd + (p.K >> 5),
-                   (int)threadIdx.x, kI8Threads);
-    }
-    return reinterpret_cast<float*>(lds + MR * stride) + ((int)threadIdx.x >> 6) * 512;
+    q8_record_rows<MR>(p.x, p.ldx, (int)blockIdx.y * MR, p.M, p.K, step, lds, (int)threadIdx.x);
+    return reinterpret_cast<float*>(lds + MR * i8_row_bytes(p.K)) + ((int)threadIdx.x >> 6) * 512;
 }
 
 template <int FMT, int MR>
@@ -660,47 +677,152 @@ __global__ __launch_bounds__(kI8Threads) void int8_q6k256_kernel(I8Launch p) {
     if (lane == 32 && two) p.y[(int64_t)blockIdx.y * p.ldy + row0 + 1] = total;
 }
 
+// Batches at a 256 step (Q4_K, Q6_K): MR activation rows per workgroup. A wave reads its
+// two weight rows once for all of them, and the serial chains of every (activation row,
+// weight row) run side by side in one pass over the blocks: sixteen lanes of Q4_K's, 64
+// of Q6_K's at four rows, where the one-row kernels keep four and sixteen busy for the
+// same round trips. Every chain sees the one-row kernels' operations in their order.
+// Bound by the staged codes' LDS reads and the chains. Us at 4 / 8 rows:
+// Q4_K 4096->14336 40 / 73 -> 29.6 / 47.8, Q6_K 41 / 78 -> 28 / 44.
+template <int FMT>
+constexpr int block_words() {  // a block's ints and scales in LDS
+    return FMT == Q4_K ? 10 : 9;
+}
+template <int FMT>
+constexpr int slot_pitch() {  // words of 16 blocks, such that the slots' chains read different banks
+    return FMT == Q4_K ? 162 : 152;
+}
+template <int FMT>
+constexpr int block_wave_bytes(int mr) {
+    return 2 * mr * slot_pitch<FMT>() * 4;
+}
+template <int FMT, int MR>
+__global__ __launch_bounds__(kI8Threads) void int8_blocks_rows_kernel(I8Launch p) {
+    constexpr int BW = block_words<FMT>(), SP = slot_pitch<FMT>(), CH = FMT == Q4_K ? 2 : 8;
+    extern __shared__ __align__(16) uint8_t i8_lds[];
+    stage_record_rows<MR>(p, 256, i8_lds);
+    const int stride = i8_row_bytes(p.K), wave = (int)threadIdx.x >> 6, lane = (int)threadIdx.x & 63;
+    float* const buf = reinterpret_cast<float*>(i8_lds + MR * stride) + wave * (2 * MR * SP);
+    const int64_t row0 = (int64_t)blockIdx.x * kI8Rows + 2 * wave;
+    if (row0 >= p.rows) return;
+    const bool two = row0 + 1 < p.rows;
+    const int nch = p.P.nch;
+    // this lane's chain: activation row m0 + slot / 2, weight row row0 + slot % 2
+    const int chain = lane % CH, slot = lane / CH, m = (int)blockIdx.y * MR + (slot >> 1);
+    const bool whole = m >= p.M - (p.M & 3) || (p.tail && m == p.M - 1);
+    const float* const mine = buf + slot * SP;
+    float acc = 0.f;
+    for (int c0 = 0; c0 < nch; c0 += 64) {
+        const int c = c0 + lane;
+        if (c < nch) {  // whole quads: nch is a multiple of four
+            ChunkData<FMT> D[2];
+            load_chunk<FMT>(p.P, row0, c, D[0]);
+            load_chunk<FMT>(p.P, two ? row0 + 1 : row0, c, D[1]);
+#pragma unroll
+            for (int r = 0; r < MR; ++r) {
+                const int8_t* xc = reinterpret_cast<const int8_t*>(i8_lds + r * stride);
+                const float* xd = reinterpret_cast<const float*>(i8_lds + r * stride + p.K);
+#pragma unroll
+                for (int w = 0; w < 2; ++w) {
+                    if constexpr (FMT == Q4_K) q4k256_ints(D[w], c, xc, xd, buf + (2 * r + w) * SP);
+                    else q6k256_ints(D[w], c, xc, xd, buf + (2 * r + w) * SP);
+                }
+            }
+        }
+        __builtin_amdgcn_wave_barrier();
+        if (slot < 2 * MR) {
+            const int blocks = min(16, (nch - c0) >> 2);
+#pragma unroll 4
+            for (int b = 0; b < blocks; ++b) {
+                const float* blk = mine + b * BW;
+                if constexpr (FMT == Q4_K) {
+                    const float s = blk[8 + chain];
+                    int q[4];
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) q[i] = __builtin_bit_cast(int, blk[2 * i + chain]);
+                    if (whole) {
+                        acc = fmaf((float)((q[0] + q[1]) + (q[2] + q[3])), s, acc);
+                    } else {
+#pragma unroll
+                        for (int i = 0; i < 4; ++i) acc = fmaf((float)q[i], s, acc);
+                    }
+                } else {
+                    acc = fmaf(blk[8], (float)__builtin_bit_cast(int, blk[chain]), acc);
+                }
+            }
+        }
+        __builtin_amdgcn_wave_barrier();
+    }
+    float v;
+    if constexpr (FMT == Q4_K) {
+        v = acc - lane_xor<1>(acc);
+    } else {
+        const float t = acc + lane_xor<4>(acc);
+        const float u = t + lane_xor<2>(t);
+        v = u + lane_xor<1>(u);
+    }
+    if (chain == 0 && slot < 2 * MR && m < p.M && (two || !(slot & 1))) p.y[(int64_t)m * p.ldy + row0 + (slot & 1)] = v;
+}
+
 // The records of one row, staged as the products stage them, then copied out.
 __global__ __launch_bounds__(kI8Threads) void q8_records_kernel(const float* x, int K, int step, float* d,
                                                                 int8_t* codes) {
     extern __shared__ __align__(16) uint8_t i8_lds[];
     int8_t* xc = reinterpret_cast<int8_t*>(i8_lds);
     float* xd = reinterpret_cast<float*>(i8_lds + K);
-    q8_records(x, K, step, xd, xc, xd + (K >> 5), (int)threadIdx.x, kI8Threads);
+    q8_record_rows<1>(x, 0, 0, 1, K, step, i8_lds, (int)threadIdx.x);
     for (int i = (int)threadIdx.x; i < K; i += kI8Threads) codes[i] = xc[i];
     for (int i = (int)threadIdx.x; i < (K >> 5); i += kI8Threads) d[i] = xd[i];
 }
 
 }  // namespace
 
-// codes, steps, per-step inverses (rounded up to 16 bytes), then 2 KiB of
+// codes, steps, spare words (rounded up to 16 bytes), then 2 KiB of
 // slice values per wave.
 size_t int8_lds_bytes(int64_t cols) {
     const size_t tail = (size_t)(cols / 32) + (size_t)((cols + 255) / 256);
     return (size_t)cols + ((tail + 3) & ~size_t(3)) * 4 + (size_t)(kI8Threads / 64) * 2048;
 }
 
-// Activation rows per workgroup of a Q8_0 batch: four from eight rows, two from four,
-// where their records fit 64 KiB of LDS. RQMV_I8_ROWS=1/2/4 overrides it for tuning.
-static int int8_rows(int M, int K) {
+// Activation rows per workgroup of a batch: four from four rows and two from two, where
+// that leaves two workgroups per CU (Q8_0 5120x5120 at four rows 14.3 us alone, 13.1 by
+// twos, 15.9 by fours; Q4_K 1111x2048 at four 6.6 / 6.5 / 8.3) and their records and the
+// waves' buffers fit 64 KiB of LDS. Three and five rows would leave a third of the places
+// empty, and run alone. RQMV_I8_ROWS=1/2/4 overrides it for tuning.
+static int int8_rows(int M, int64_t rows, int K, size_t (*wave_bytes)(int)) {
+    const int64_t tiles = (rows + kI8Rows - 1) / kI8Rows;
+    int mr = 1;
+    if (M >= 2 && M != 3 && M != 5) mr = M >= 4 && tiles * ((M + 3) / 4) >= 512 ? 4 : tiles * ((M + 1) / 2) >= 512 ? 2 : 1;
     const char* env = getenv("RQMV_I8_ROWS");
-    const int want = env && *env ? atoi(env) : M >= 8 ? 4 : M >= 4 ? 2 : 1;
-    int mr = want >= 4 ? 4 : want >= 2 ? 2 : 1;
-    while (mr > 1 && (size_t)mr * i8_row_bytes(K) + (size_t)(kI8Threads / 64) * 2048 > 65536) mr >>= 1;
+    if (env && *env) mr = atoi(env) >= 4 ? 4 : atoi(env) >= 2 ? 2 : 1;
+    while (mr > 1 && (size_t)mr * i8_row_bytes(K) + (size_t)(kI8Threads / 64) * wave_bytes(mr) > 65536) mr >>= 1;
     return mr;
 }
 
 template <int FMT>
+static hipError_t launch_blocks(const I8Launch& p, hipStream_t stream) {
+    auto wave_bytes = [](int mr) -> size_t { return block_wave_bytes<FMT>(mr); };
+    const int mr = int8_rows(p.M, p.rows, p.K, wave_bytes);
+    const dim3 grid((unsigned)((p.rows + kI8Rows - 1) / kI8Rows), (unsigned)((p.M + mr - 1) / mr));
+    size_t lds = int8_lds_bytes(p.K);
+    void (*kernel)(I8Launch) = FMT == Q4_K ? int8_q4k256_kernel : int8_q6k256_kernel;
+    if (mr > 1) {
+        lds = (size_t)mr * i8_row_bytes(p.K) + (size_t)(kI8Threads / 64) * wave_bytes(mr);
+        kernel = mr == 4 ? int8_blocks_rows_kernel<FMT, 4> : int8_blocks_rows_kernel<FMT, 2>;
+    }
+    hipLaunchKernelGGL(kernel, grid, dim3(kI8Threads), lds, stream, p);
+    return hipGetLastError();
+}
+
+template <int FMT>
 static hipError_t launch_slices(const I8Launch& p, hipStream_t stream) {
-    const int mr = FMT == Q8_0 ? int8_rows(p.M, p.K) : 1;
+    const int mr = int8_rows(p.M, p.rows, p.K, [](int) -> size_t { return 2048; });
     const dim3 grid((unsigned)((p.rows + kI8Rows - 1) / kI8Rows), (unsigned)((p.M + mr - 1) / mr));
     size_t lds = int8_lds_bytes(p.K);
     auto kernel = int8_slices_kernel<FMT>;
-    if constexpr (FMT == Q8_0) {
-        if (mr > 1) {
-            lds = (size_t)mr * i8_row_bytes(p.K) + (size_t)(kI8Threads / 64) * 2048;
-            kernel = mr == 4 ? int8_slices_rows_kernel<FMT, 4> : int8_slices_rows_kernel<FMT, 2>;
-        }
+    if (mr > 1) {
+        lds = (size_t)mr * i8_row_bytes(p.K) + (size_t)(kI8Threads / 64) * 2048;
+        kernel = mr == 4 ? int8_slices_rows_kernel<FMT, 4> : int8_slices_rows_kernel<FMT, 2>;
     }
     hipLaunchKernelGGL(kernel, grid, dim3(kI8Threads), lds, stream, p);
     return hipGetLastError();
@@ -709,17 +831,8 @@ static hipError_t launch_slices(const I8Launch& p, hipStream_t stream) {
 hipError_t launch_matvec_int8(int fmt, const Planes& P, int64_t rows, int K, const float* x, int M, int64_t ldx,
                               float* y, int64_t ldy, int step, int tail, hipStream_t stream) {
     I8Launch p{P, rows, K, x, ldx, y, ldy, M, step, tail};
-    const dim3 grid((unsigned)((rows + kI8Rows - 1) / kI8Rows), (unsigned)M);
-    const size_t lds = int8_lds_bytes(K);
-    const bool blocks256 = step == 256 && (fmt == Q4_K || fmt == Q6_K);
-    if (blocks256 && fmt == Q4_K) {
-        hipLaunchKernelGGL(int8_q4k256_kernel, grid, dim3(kI8Threads), lds, stream, p);
-        return hipGetLastError();
-    }
-    if (blocks256) {
-        hipLaunchKernelGGL(int8_q6k256_kernel, grid, dim3(kI8Threads), lds, stream, p);
-        return hipGetLastError();
-    }
+    if (step == 256 && fmt == Q4_K) return launch_blocks<Q4_K>(p, stream);
+    if (step == 256 && fmt == Q6_K) return launch_blocks<Q6_K>(p, stream);
     switch (fmt) {
         case Q4_K: return launch_slices<Q4_K>(p, stream);
         case Q6_K: return launch_slices<Q6_K>(p, stream);

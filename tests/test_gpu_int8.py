@@ -172,3 +172,18 @@ def test_q8_0_batches_by_rows_per_workgroup(gpu, mr, step, monkeypatch):
         got = gpu.contract_int8(W, x, step)
         want = oracle.int8_matvec("q8_0", w, rows, cols, x, step)
         assert np.array_equal(np.asarray(got, np.float32).view(np.uint32), np.asarray(want, np.float32).view(np.uint32))
+
+
+@pytest.mark.parametrize("fmt", ["q4_k", "q6_k", "q4_0"])
+@pytest.mark.parametrize("step", [32, 256])
+@pytest.mark.parametrize("mr", ["1", "2", "4"])
+def test_batches_by_rows_per_workgroup(gpu, mr, step, fmt, monkeypatch):
+    """Batches of the other formats with one, two and four activation rows per
+    workgroup: whole and partial groups (the batch's last M % 4 rows by whole blocks),
+    one row of a pair, partial passes, and rows too long for four records in LDS."""
+    monkeypatch.setenv("RQMV_I8_ROWS", mr)
+    for rows, cols, m in ((35, 256, 3), (16, 4352, 7), (1, 4096, 9), (18, 14336, 4)):
+        w = synth.weights(fmt, rows, cols, seed=rows)
+        x = np.stack([synth.activations_f32(cols, seed=50 + i) for i in range(m)])
+        W = gpu.Weight(fmt, rows, cols, w)
+        assert _bits_equal(gpu.contract_int8(W, x, step), oracle.int8_matvec(fmt, w, rows, cols, x, step)), (rows, cols, m)
