@@ -106,8 +106,9 @@ __device__ __forceinline__ uint4 ld16_nt(const uint8_t* p) {
 
 // Loads chunk c of physical row `row`. Offsets are 32-bit (a weight is smaller
 // than 4 GiB, which the loader checks), so the loads take a scalar base
-// address plus one VGPR offset each.
-template <int FMT>
+// address plus one VGPR offset each. NT: the codes as non-temporal loads, for
+// weights that nothing reads again soon.
+template <int FMT, bool NT = true>
 __device__ __forceinline__ void load_chunk(const Planes& P, int64_t row, int c, ChunkData<FMT>& d) {
     constexpr int QP = Traits<FMT>::QP;
     const uint32_t group = (uint32_t)c >> 6, within = (uint32_t)c & 63u;
@@ -115,7 +116,10 @@ __device__ __forceinline__ void load_chunk(const Planes& P, int64_t row, int c, 
     const uint32_t nb = rest > 64u ? 64u : rest;
     const uint32_t gb = (uint32_t)row * (uint32_t)P.row_bytes + group * full_group_bytes<FMT>();
 #pragma unroll
-    for (int h = 0; h < QP; ++h) d.q[h] = ld16_nt(P.base + (gb + ((uint32_t)h * nb + within) * 16u));
+    for (int h = 0; h < QP; ++h) {
+        const uint8_t* const at = P.base + (gb + ((uint32_t)h * nb + within) * 16u);
+        d.q[h] = NT ? ld16_nt(at) : ld16(at);
+    }
     const uint32_t meta = gb + (uint32_t)QP * nb * 16u;
     if constexpr (FMT == Q4_K) {
         d.meta = ld16(P.base + (meta + (within >> 2) * 16u));

@@ -25,7 +25,7 @@
 namespace rq {
 
 constexpr int kMoeThreads = 256;  // workgroup size of the MoE kernels (four waves)
-constexpr int kMoeDownBatchMin = 16;  // positions from which the down product takes the batch form
+constexpr int kMoeBatchMin = 16;  // positions from which the products take their batch forms
 constexpr int kMoeOwnRouteMax = 2;  // positions per launch up to which every wave routes on its own
 
 static size_t al(size_t v) { return (v + 255) & ~size_t(255); }
@@ -266,12 +266,20 @@ __device__ __forceinline__ void route_wave(const MoeDims& d, const MoeWorkspace&
 template <int FMT, bool XF32, int S, bool RING, bool GSPLIT = false>
 __global__ void __launch_bounds__(kMoeThreads) moe_glu_kernel(MoeDims d, MoeBank gate, MoeBank up, MoeBank gate_sh,
                                                        MoeBank up_sh, const void* x, MoeWorkspace ws, float* route_dense,
-                                                       int G, MoeBatch batch) {
+                                                       int G, MoeBatch batch, int blocks) {
     constexpr int XP = Traits<FMT>::XP;
-    // position blockIdx.y of the batch
-    x = static_cast<const char*>(x) + batch.x_stride * blockIdx.y;
-    ws = position_ws(ws, batch.ws_stride, (int)blockIdx.y);
-    if (route_dense) route_dense += batch.route_stride * blockIdx.y;
+    // position blockIdx.y of the batch, or (blocks > 0) the position and the block
+    // of rows that the workgroup's place on its XCD gives
+    int pos = (int)blockIdx.y, block = (int)blockIdx.x;
+    if (RING && blocks) {
+        const int j8 = (int)blockIdx.x >> 3;
+        pos = j8 % batch.m;
+        block = ((int)blockIdx.x & 7) + 8 * (j8 / batch.m);
+        if (block >= blocks) return;
+    }
+    x = static_cast<const char*>(x) + batch.x_stride * pos;
+    ws = position_ws(ws, batch.ws_stride, pos);
+    if (route_dense) route_dense += batch.route_stride * pos;
     extern __shared__ uint4 smem[];
     __shared__ int slot_ids_all[4][64];
     const int nch = gate.P.nch;
@@ -280,8 +288,12 @@ __global__ void __launch_bounds__(kMoeThreads) moe_glu_kernel(MoeDims d, MoeBank
     const int lane = threadIdx.x & 63, g = lane & (G - 1), sub = lane / G;
     const int wpb = kMoeThreads >> 6, wave = threadIdx.x >> 6;
     const int routed = d.top * d.hidden;
-    const int total_rows = routed + d.hidden_shared;
     const int rows_per_wave = 64 / G;
+    // (blocks > 0: rows block * span .. of every routed slot, then the shared expert's)
+    const bool blocked = RING && blocks > 0;
+    const int span = blocked ? (d.hidden + blocks - 1) / blocks : d.hidden;
+    const int span_sh = blocked ? (d.hidden_shared + blocks - 1) / blocks : d.hidden_shared;
+    const int routed_span = d.top * span, total_rows = routed_span + span_sh;
     const int tiles = (total_rows + rows_per_wave - 1) / rows_per_wave;
     // The position is routed here (a few microseconds of one wave, instead of
     // a launch and a round trip through memory); the first wave of the first
@@ -295,24 +307,40 @@ __global__ void __launch_bounds__(kMoeThreads) moe_glu_kernel(MoeDims d, MoeBank
     const bool multi = stage_items<FMT>(nch, 1) <= kStageNJ * kMoeThreads;
     StageItem<XF32> it[kStageNJ];
     if (multi) stage_multi_issue<FMT, XF32>(nch, d.d_model, x, 0, 1, kMoeThreads, it);
-    if (!RING || wave == 0) route_wave<S>(d, ws, route_dense, blockIdx.x == 0 && wave == 0, slot_ids);
+    if (!RING || wave == 0) route_wave<S>(d, ws, route_dense, block == 0 && wave == 0, slot_ids);
     if constexpr (RING) __syncthreads();
-    // Row r of the gate/up stack: hidden row f of routed slot s, or of the shared expert.
+    // Row r of the workgroup's gate/up rows: hidden row f of routed slot s, or of the
+    // shared expert (its place in ws.h: h_row; -1 past the expert's rows).
+    const int first = blocked ? block * span : 0, first_sh = blocked ? block * span_sh : 0;
+    auto h_row = [&](int r) -> int {
+        if (r >= total_rows) return -1;
+        if (!blocked) return r;
+        if (r < routed_span) {
+            const int s = r / span, f = first + r % span;
+            return f < d.hidden ? s * d.hidden + f : -1;
+        }
+        const int f = first_sh + r - routed_span;
+        return f < d.hidden_shared ? routed + f : -1;
+    };
     auto fetch = [&](int r, int c, ChunkData<FMT>& dg, ChunkData<FMT>& du) {
         r = r < total_rows ? r : total_rows - 1;
         c = c < nch ? c : nch - 1;
-        if (r < routed) {
-            const int s = r / d.hidden, f = r % d.hidden;
+        if (r < routed_span) {
+            const int s = r / span;
+            int f = first + r % span;
+            f = f < d.hidden ? f : d.hidden - 1;
             const int64_t e = slot_ids[s];
-            load_chunk<FMT>(gate.P, e * gate.rows + f, c, dg);
-            load_chunk<FMT>(up.P, e * up.rows + f, c, du);
+            load_chunk<FMT, !RING>(gate.P, e * gate.rows + f, c, dg);
+            load_chunk<FMT, !RING>(up.P, e * up.rows + f, c, du);
         } else {
-            load_chunk<FMT>(gate_sh.P, r - routed, c, dg);
-            load_chunk<FMT>(up_sh.P, r - routed, c, du);
+            int f = first_sh + r - routed_span;
+            f = f < d.hidden_shared ? f : d.hidden_shared - 1;
+            load_chunk<FMT, !RING>(gate_sh.P, f, c, dg);
+            load_chunk<FMT, !RING>(up_sh.P, f, c, du);
         }
     };
-    int tile = blockIdx.x * wpb + wave;
-    const int stride = gridDim.x * wpb;
+    int tile = blocked ? wave : (int)blockIdx.x * wpb + wave;
+    const int stride = blocked ? wpb : (int)gridDim.x * wpb;
     // the first tile's weights are requested before the activations are staged
     ChunkData<FMT> dg0, du0, dg1, du1;
     fetch((tile < tiles ? tile : tiles - 1) * rows_per_wave + sub, g, dg0, du0);
@@ -411,7 +439,8 @@ __global__ void __launch_bounds__(kMoeThreads) moe_glu_kernel(MoeDims d, MoeBank
         }
         ag = group_sum(ag, G);
         au = group_sum(au, G);
-        if (r < total_rows && g == G - 1) ws.h[r] = act_apply_likely_silu(d.activation, d.act_factor, ag) * au;
+        const int at = h_row(r);
+        if (at >= 0 && g == G - 1) ws.h[at] = act_apply_likely_silu(d.activation, d.act_factor, ag) * au;
     };
     while (tile < tiles) {
         step(tile, dg0, du0, dg1, du1);
@@ -812,8 +841,39 @@ static hipError_t glu_launch(const MoeDims& d, const MoeBank& gate, const MoeBan
                                            hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
         if (e != hipSuccess) return e;
     }
-    hipLaunchKernelGGL(kernel, dim3(grid, b.m), dim3(kMoeThreads), lds, stream, d, gate, up, gate_sh, up_sh, x, ws,
-                       route_dense, GL, b);
+    // From 16 positions, a workgroup takes one position's rows of one block of the hidden
+    // width, and an XCD passes all positions over a block before the next, so that the
+    // positions that chose an expert find its rows in the XCD's L2 or close to it; weights
+    // are read with ordinary loads (non-temporal ones mark their lines for early eviction).
+    // gguf_moe workload, us per step at 16 / 64 / 512 positions: 71 / 161 / 1018 with the
+    // form below 16 positions and its non-temporal loads, 68 / 161 / 950 with ordinary
+    // loads -> 65 / 150 / 841 in 32 blocks (16 blocks 77 / 155 / 859, 64 blocks 65 / 154 /
+    // 877); Q8_0, hidden 256, top 4, 300 positions 260 -> 162 in 16, Q6_K, hidden 768, top
+    // 6 and shared, 100 positions 447 -> 323 in 48. Workgroups of about 144 rows measured
+    // best, at least 16 blocks (Q8_0, hidden 256, top 2 and shared, 512 positions: 8 / 16 /
+    // 32 blocks 246 / 235 / 245), and more where there would be less than 1024 workgroups
+    // (Q6_K, hidden 768, 16 positions: 16 / 32 / 64 blocks 101 / 92 / 89). Banks that the
+    // eight L2s hold whole (32 MB) gain nothing (Q4_K, 32 experts of 256, 512 positions: 79
+    // us striding, 86 in 8 blocks). RQMV_MOE_GLU_BLOCKS overrides the count, 0 for the
+    // striding form.
+    const char* benv = getenv("RQMV_MOE_GLU_BLOCKS");
+    int blocks = 0;
+    if (b.m >= kMoeBatchMin && (benv && *benv)) blocks = atoi(benv);
+    else if (b.m >= kMoeBatchMin && (int64_t)gate.P.bytes + (int64_t)up.P.bytes > (32 << 20)) {
+        const int by_rows = total_rows > 16 * 144 ? (total_rows + 143) / 144 : 16, by_fill = (1024 + b.m - 1) / b.m;
+        blocks = ((by_rows > by_fill ? by_rows : by_fill) + 7) / 8 * 8;
+        if (blocks > (d.hidden + 7) / 8) blocks = (d.hidden + 7) / 8;
+    }
+    if (blocks > d.hidden) blocks = d.hidden;
+    if (blocks > 0) {
+        const int64_t wgs = (int64_t)((blocks + 7) / 8 * 8) * b.m;
+        if (wgs > 0x7FFFFFFF) return hipErrorInvalidValue;
+        hipLaunchKernelGGL(kernel, dim3((unsigned)wgs), dim3(kMoeThreads), lds, stream, d, gate, up, gate_sh, up_sh, x, ws,
+                           route_dense, GL, b, blocks);
+    } else {
+        hipLaunchKernelGGL(kernel, dim3(grid, b.m), dim3(kMoeThreads), lds, stream, d, gate, up, gate_sh, up_sh, x, ws,
+                           route_dense, GL, b, 0);
+    }
     return hipGetLastError();
 }
 
@@ -892,7 +952,7 @@ static hipError_t down_fmt(const MoeDims& d, const MoeBank& down, const MoeBank&
     // the non-temporal ones of the one-position form, which mark lines for early
     // eviction, the same steps took 50 / 74.6 / 174.8 / 1223.
     const size_t blds = (size_t)nch * (size_t)(down_pitch<FMT>() + 16);
-    if (G <= 32 && blds <= 65536 && env_flag("RQMV_MOE_DOWN_BATCH", b.m >= kMoeDownBatchMin)) {
+    if (G <= 32 && blds <= 65536 && env_flag("RQMV_MOE_DOWN_BATCH", b.m >= kMoeBatchMin)) {
         const char* senv = getenv("RQMV_MOE_DOWN_SPAN");
         const int span = senv && *senv ? atoi(senv) / 32 * 32 : b.m >= 48 ? 128 : 64;
         if (span < 32) return hipErrorInvalidValue;

@@ -60,3 +60,21 @@ def test_batches_carry_the_bits_of_single_positions(gpu, case, xdt, kind, m):
         assert np.array_equal(got[p, :d].view(np.uint32), y1.view(np.uint32)), (case, p)
         assert np.array_equal(routes[p].view(np.uint32), r1.view(np.uint32)), (case, p)
     assert (got[:, d:] == 0).all()
+
+
+@pytest.mark.parametrize("case", CASES, ids=lambda c: "-".join(map(str, c)))
+@pytest.mark.parametrize("blocks", ["0", "5", "16"])
+def test_gate_up_by_blocks_of_rows(gpu, case, blocks, monkeypatch):
+    """The gate/up product striding over a position's rows and by blocks of the hidden
+    width: blocks that divide it, and blocks that leave partial and empty ones."""
+    monkeypatch.setenv("RQMV_MOE_GLU_BLOCKS", blocks)
+    d, m = case[1], 18
+    moe = _moe(gpu, case, seed=sum(case[1:6]))
+    x = _activations(m, d, "f32", "outliers", seed=m + d)
+    y = gpu.DeviceBuffer(4 * m * d)
+    y.fill_zero()
+    moe.run_batch(gpu.DeviceBuffer.from_array(x), gpu.DTYPE_F32, m, d, y, d, None, moe.batch_workspace(m))
+    gpu.synchronize()
+    got = y.download(np.float32).reshape(m, d)
+    for p in range(m):
+        assert np.array_equal(got[p].view(np.uint32), moe(x[p])[0].view(np.uint32)), (case, p)
