@@ -144,8 +144,8 @@ __host__ __device__ inline int i8_row_bytes(int K) {
 // (amd-nv-cpu.ll:1408-1440): 32 lanes per step each hold those inputs, take the extreme
 // over the lanes by exchanges and code what they hold. With one thread per (step, lane), then one per
 // step over 32 LDS reads, then one per record, a row's records took about 3 us of a
-// workgroup: Q4_K 1111x2048, one and two rows 6.6 -> 5.3 us, Q6_K 14336 x 4096 at
-// eight rows, a workgroup a row, 78 -> 70.
+// workgroup: Q4_K 1111x2048 at two rows 6.6 -> 4.8 us, Q6_K 14336 x 4096 at
+// eight rows, a workgroup a row, 78 -> 61.
 template <int MR>
 __device__ __forceinline__ void q8_record_rows(const float* __restrict__ x, int64_t ldx, int m0, int M, int K, int step,
                                                uint8_t* lds, int tid) {
@@ -683,7 +683,7 @@ __global__ __launch_bounds__(kI8Threads) void int8_q6k256_kernel(I8Launch p) {
 // of Q6_K's at four rows, where the one-row kernels keep four and sixteen busy for the
 // same round trips. Every chain sees the one-row kernels' operations in their order.
 // Bound by the staged codes' LDS reads and the chains. Us at 4 / 8 rows:
-// Q4_K 4096->14336 40 / 73 -> 29.6 / 47.8, Q6_K 41 / 78 -> 28 / 44.
+// Q4_K 4096->14336 31 / 58 -> 26.4 / 43.6, Q6_K 32 / 61 -> 23 / 37.
 template <int FMT>
 constexpr int block_words() {  // a block's ints and scales in LDS
     return FMT == Q4_K ? 10 : 9;
