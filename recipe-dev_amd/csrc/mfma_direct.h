@@ -10,11 +10,11 @@
 // registers. A lane (row m, slice kq) loads the eight activations its A
 // operand holds, PD operands ahead.
 //
-// fp32 activations become two fp16 operands per 32-value block: the block is
-// scaled by the power of two 2^k that brings its largest magnitude into
-// [2^14, 2^15) and split into a high and a low part (x = hi + lo to 2^-22 of
-// the value); the block's scale times 2^-k multiplies the sum of the two
-// products in fp32. Up to eight activation rows (PACK), the high parts are
+// fp32 activations become two fp16 operands per 32-value block: the block (Q6_K:
+// each of its two 16-value scale groups) is scaled by the power of two 2^k that
+// brings its largest magnitude into [2^14, 2^15) and split into a high and a low
+// part (x = hi + lo to 2^-22 of the value); its scale times 2^-k multiplies the
+// sum of the two products in fp32. Up to eight activation rows (PACK), the high parts are
 // rows 0-7 of one A operand and the low parts rows 8-15: the same count of
 // matrix-core products as fp16 activations, the two halves added at the end.
 //
@@ -27,8 +27,8 @@
 // repeats (about 45 instructions per eight values), and at few rows the round
 // trips of a wave's two or four steps; the weights' bytes take a fifth of the
 // time. Measured against the staged form this replaces (kernel us, fp32 x): Q4_K
-// 4096x4096 at 5 rows 83.8 -> 13.1 (720 GB/s), Q6_K 14336->4096 at 77 rows
-// 3363 -> 107 (85 TFLOP/s).
+// 4096x4096 at 5 rows 83.8 -> 12.2 (780 GB/s), Q6_K 14336->4096 at 77 rows
+// 3363 -> 114 (79 TFLOP/s).
 #pragma once
 
 #include <hip/hip_ext.h>
@@ -78,15 +78,24 @@ __device__ __forceinline__ uint32_t opaque(uint32_t v) {
 // held in registers until then.
 __device__ __forceinline__ void pin(f4_t& v) { asm volatile("" : "+v"(v)); }
 
-// The largest of a value over the four lanes 16 apart, in each of them.
-__device__ __forceinline__ float max_over_slices(float v) {
+// The largest of a value over slices 0 and 1, or 2 and 3 (the lanes 16 apart that
+// hold one scale group of Q6_K), in both.
+__device__ __forceinline__ float max_over_pair(float v) {
     uint32_t a = __builtin_bit_cast(uint32_t, v), b = opaque(a);
     swap_bit4(a, b);
-    v = fmaxf(__builtin_bit_cast(float, a), __builtin_bit_cast(float, b));
-    a = __builtin_bit_cast(uint32_t, v);
-    b = opaque(a);
-    swap_bit5(a, b);
     return fmaxf(__builtin_bit_cast(float, a), __builtin_bit_cast(float, b));
+}
+// Both pairs' largest, in all four lanes.
+__device__ __forceinline__ void pair_maxima(float v, float& first, float& second) {
+    uint32_t a = __builtin_bit_cast(uint32_t, max_over_pair(v)), b = opaque(a);
+    swap_bit5(a, b);
+    first = __builtin_bit_cast(float, a);
+    second = __builtin_bit_cast(float, b);
+}
+__device__ __forceinline__ float max_over_slices(float v) {
+    float a, b;
+    pair_maxima(v, a, b);
+    return fmaxf(a, b);
 }
 
 // Lane i of 16-lane row kq takes lane (i + 4 kq) mod 16 of a value that every
@@ -205,6 +214,16 @@ __device__ __forceinline__ h8_t direct_operand(const DirectWords<FMT>& w, int b,
     return __builtin_bit_cast(h8_t, make_uint4(o[0], o[1], o[2], o[3]));
 }
 
+// Q6_K: a block's weights with those of the other scale group (first: slices 0 and
+// 1) zero. A product per group, each scaled on its own: the second group's sum as
+// the whole block's less the first's would keep the first's rounding, however small
+// its scale (one value of 1e5 in a group of scale 0 beside one of scale 100, 4096
+// columns: error against 64 bits 6e-5 instead of 3e-7).
+__device__ __forceinline__ h8_t group_operand(const h8_t& B, bool mine) {
+    const uint4 o = __builtin_bit_cast(uint4, B);
+    return __builtin_bit_cast(h8_t, make_uint4(mine ? o.x : 0u, mine ? o.y : 0u, mine ? o.z : 0u, mine ? o.w : 0u));
+}
+
 // Sub-block `b` (0..7) of a Q4_K superblock: its six-bit scale and minimum, for
 // an index known at compile time (one funnel shift per 24-bit field).
 __device__ __forceinline__ void q4k_scale_min(const uint4& meta, int b, uint32_t& sc, uint32_t& mn) {
@@ -217,8 +236,8 @@ __device__ __forceinline__ void q4k_scale_min(const uint4& meta, int b, uint32_t
     mn = bfe(f, 12 * (b & 1) + 6, 6);
 }
 
-// Row n's scales of block b of a step: s0 (Q6_K: the second 16-value group's),
-// s1 (Q4_K: the minimum; Q6_K: the first group's minus the second's). Chunks
+// Row n's scales of block b of a step: s0 (Q6_K: the first 16-value group's),
+// s1 (Q4_K: the minimum; Q6_K: the second group's). Chunks
 // past the row's end scale by zero (the bytes there are not the row's).
 template <int FMT>
 __device__ __forceinline__ void direct_scales(const DirectStep<FMT>& t, int b, bool chunk_ok, float& s0, float& s1) {
@@ -241,10 +260,8 @@ __device__ __forceinline__ void direct_scales(const DirectStep<FMT>& t, int b, b
     } else {
         const uint32_t scw = word(t.meta, c);
         const float dd = half_lo(t.d);
-        const float g0 = dd * (float)(int8_t)((scw >> (16 * sub)) & 0xffu);
-        const float g1 = dd * (float)(int8_t)((scw >> (16 * sub + 8)) & 0xffu);
-        s0 = g1;
-        s1 = g0 - g1;
+        s0 = dd * (float)(int8_t)((scw >> (16 * sub)) & 0xffu);
+        s1 = dd * (float)(int8_t)((scw >> (16 * sub + 8)) & 0xffu);
     }
 }
 
@@ -324,15 +341,14 @@ __global__ void __launch_bounds__(64 * kDirectMaxWaves) matvec_mfma_direct(MvPar
         for (int r = 0; r < RT; ++r) direct_words<FMT>(cur[r], lane, wd[r]);
 #pragma unroll
         for (int b = 0; b < NB; ++b) {
-            h8_t B[RT], B0[RT];
+            h8_t B[RT], B1[RT];  // (Q6_K: the first and the second scale group's)
             float s0[RT], s1[RT];
 #pragma unroll
             for (int r = 0; r < RT; ++r) {
                 B[r] = direct_operand<FMT>(wd[r], b, kq);
                 if constexpr (FMT == Q6_K) {
-                    const uint4 o = __builtin_bit_cast(uint4, B[r]);
-                    const bool g0 = kq < 2;  // the block's first scale group
-                    B0[r] = __builtin_bit_cast(h8_t, make_uint4(g0 ? o.x : 0u, g0 ? o.y : 0u, g0 ? o.z : 0u, g0 ? o.w : 0u));
+                    B1[r] = group_operand(B[r], kq >= 2);
+                    B[r] = group_operand(B[r], kq < 2);
                 }
                 direct_scales<FMT>(cur[r], b, 4 * s + b / BPC < nch, s0[r], s1[r]);
             }
@@ -347,17 +363,32 @@ __global__ void __launch_bounds__(64 * kDirectMaxWaves) matvec_mfma_direct(MvPar
                     v[e] = __builtin_bit_cast(float, word(a.v[0], e));
                     v[4 + e] = __builtin_bit_cast(float, word(a.v[1], e));
                 }
-                // the block's largest magnitude (a NaN takes the zero shift's way
-                // through the split, as an infinity does)
+                // the block's (Q6_K: each scale group's) largest magnitude (a NaN
+                // takes the zero shift's way through the split, as an infinity does)
                 float am = 0.f;
 #pragma unroll
                 for (int e = 0; e < 8; ++e) am = fmaxf(am, fabsf(v[e]));
-                am = max_over_slices(am);
-                const int ks = block_shift(am);
                 uint32_t hi[4], lo[4];
-                split_hi_lo(v, pow2f(ks), hi, lo);
-                const float fx = rotate_to_rows(pow2f(-ks));
-                const float f0 = row_bcast<0>(fx), f1 = row_bcast<1>(fx), f2 = row_bcast<2>(fx), f3 = row_bcast<3>(fx);
+                float f[4], g[4];  // the inverse powers of rows 4 kq + j (g: the second group's)
+                auto rows_of = [](int k, float (&o)[4]) {
+                    const float fx = rotate_to_rows(pow2f(-k));
+                    o[0] = row_bcast<0>(fx);
+                    o[1] = row_bcast<1>(fx);
+                    o[2] = row_bcast<2>(fx);
+                    o[3] = row_bcast<3>(fx);
+                };
+                if constexpr (FMT == Q6_K) {
+                    float am0, am1;
+                    pair_maxima(am, am0, am1);
+                    const int k0 = block_shift(am0), k1 = block_shift(am1);
+                    split_hi_lo(v, pow2f(kq < 2 ? k0 : k1), hi, lo);
+                    rows_of(k0, f);
+                    rows_of(k1, g);
+                } else {
+                    const int ks = block_shift(max_over_slices(am));
+                    split_hi_lo(v, pow2f(ks), hi, lo);
+                    rows_of(ks, f);
+                }
                 h8_t A[2];
                 if constexpr (PACK) {
                     const bool low = mn >= 8;
@@ -377,26 +408,20 @@ __global__ void __launch_bounds__(64 * kDirectMaxWaves) matvec_mfma_direct(MvPar
                 if constexpr (FMT == Q4_K) {  // the block's activation sums, unscaled
                     const h8_t one = {1, 1, 1, 1, 1, 1, 1, 1};
                     bs = product(one);
-                    bs[0] *= f0;
-                    bs[1] *= f1;
-                    bs[2] *= f2;
-                    bs[3] *= f3;
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) bs[j] *= f[j];
                 }
 #pragma unroll
                 for (int r = 0; r < RT; ++r) {
                     const f4_t D = product(B[r]);
                     f4_t& ac = acc[r][t];
                     if constexpr (FMT == Q6_K) {
-                        const f4_t D0 = product(B0[r]);
-                        ac[0] = fmaf(s1[r] * f0, D0[0], ac[0]);
-                        ac[1] = fmaf(s1[r] * f1, D0[1], ac[1]);
-                        ac[2] = fmaf(s1[r] * f2, D0[2], ac[2]);
-                        ac[3] = fmaf(s1[r] * f3, D0[3], ac[3]);
+                        const f4_t D1 = product(B1[r]);
+#pragma unroll
+                        for (int j = 0; j < 4; ++j) ac[j] = fmaf(s1[r] * g[j], D1[j], ac[j]);
                     }
-                    ac[0] = fmaf(s0[r] * f0, D[0], ac[0]);
-                    ac[1] = fmaf(s0[r] * f1, D[1], ac[1]);
-                    ac[2] = fmaf(s0[r] * f2, D[2], ac[2]);
-                    ac[3] = fmaf(s0[r] * f3, D[3], ac[3]);
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) ac[j] = fmaf(s0[r] * f[j], D[j], ac[j]);
                     if constexpr (FMT == Q4_K) {
 #pragma unroll
                         for (int j = 0; j < 4; ++j) ac[j] = fmaf(-s1[r], bs[j], ac[j]);

@@ -18,10 +18,10 @@
 // the block's d scales the tile once per 256 weights. Q4_K's minimums are one
 // more product per 256 weights, of the eight 6-bit minimums with the eight
 // sub-blocks' activation sums, each sum as three bf16 parts (24 bits).
-// Otherwise every 32-weight block is a product of its own, scaled in fp32 into
-// the sums (fp32 activations: high and low fp16 parts as in mfma_direct.h, the
-// block's power of two times its scale; Q4_K's minimum times the block's fp32
-// activation sum).
+// Otherwise every 32-weight block (Q6_K: each 16-weight scale group) is a product
+// of its own, scaled in fp32 into the sums (fp32 activations: high and low fp16 parts
+// as in mfma_direct.h, the power of two times the scale; Q4_K's minimum times the
+// block's fp32 activation sum).
 //
 // Bound. At 512 rows, VALU issue (the scaled sums, four fmas per product, and the
 // decode) beside the products with two waves per SIMD: the matrix cores are busy for
@@ -41,7 +41,8 @@ struct TileCfg {
     static constexpr int XN = XF32 ? 2 : 1;                 // operands per activation tile
     static constexpr int WB = 4;                            // 32-value blocks per window
     static constexpr int ABYTES = WB * MT * XN * 1024;      // a window's operands
-    static constexpr int FBYTES = XF32 ? WB * MT * 64 : 0;  // fp32 x: a power of two per (block, row)
+    static constexpr int GS = FMT == Q6_K ? 2 : 1;          // scale groups per block
+    static constexpr int FBYTES = XF32 ? WB * MT * GS * 64 : 0;  // fp32 x: a power of two per (group, row)
     static constexpr int SBYTES = XF32 && FMT == Q4_K ? WB * MT * 64 : 0;  // fp32 x: activation sums per (block, row)
     static constexpr int BUF = ABYTES + FBYTES + SBYTES;
     static constexpr int SUMS = FOLD && FMT == Q4_K ? MT * 1024 : 0;  // Q4_K FOLD: the sums' operands, two buffers
@@ -153,14 +154,15 @@ __global__ void __launch_bounds__(64 * WN * WK) __attribute__((amdgpu_waves_per_
                 float am = 0.f;
 #pragma unroll
                 for (int e = 0; e < 8; ++e) am = fmaxf(am, fabsf(v[e]));
-                const int ks = block_shift(max_over_slices(am));
+                const int ks = block_shift(C::GS == 2 ? max_over_pair(am) : max_over_slices(am));
                 uint32_t hi[4], lo[4];
                 split_hi_lo(v, pow2f(ks), hi, lo);
                 const uint4 h4 = make_uint4(hi[0], hi[1], hi[2], hi[3]), l4 = make_uint4(lo[0], lo[1], lo[2], lo[3]);
                 *reinterpret_cast<uint4*>(buf + (2 * f) * 1024 + lane * 16) = h4;
                 *reinterpret_cast<uint4*>(buf + (2 * f + 1) * 1024 + lane * 16) = l4;
                 const float fx = pow2f(-ks);
-                if (kq == 0) *reinterpret_cast<float*>(buf + C::ABYTES + f * 64 + mn * 4) = fx;
+                if (kq % (4 / C::GS) == 0)
+                    *reinterpret_cast<float*>(buf + C::ABYTES + (C::GS * f + kq / (4 / C::GS)) * 64 + mn * 4) = fx;
                 if constexpr (FMT == Q4_K) {
                     f4_t sum = __builtin_amdgcn_mfma_f32_16x16x32_f16(ones, __builtin_bit_cast(h8_t, h4), z, 0, 0, 0);
                     sum = __builtin_amdgcn_mfma_f32_16x16x32_f16(ones, __builtin_bit_cast(h8_t, l4), sum, 0, 0, 0);
@@ -246,11 +248,12 @@ __global__ void __launch_bounds__(64 * WN * WK) __attribute__((amdgpu_waves_per_
                 h8_t a[C::XN];
                 f4_t fx, bs;
             };
+            auto power = [&](int i, int h) { return *reinterpret_cast<const f4_t*>(buf + C::ABYTES + (i * C::GS + h) * 64 + kq * 16); };
             auto read = [&](int i) {
                 Operand o;
 #pragma unroll
                 for (int h = 0; h < C::XN; ++h) o.a[h] = *reinterpret_cast<const h8_t*>(buf + (i * C::XN + h) * 1024 + lane * 16);
-                if constexpr (XF32) o.fx = *reinterpret_cast<const f4_t*>(buf + C::ABYTES + i * 64 + kq * 16);
+                if constexpr (XF32 && C::GS == 1) o.fx = power(i, 0);
                 if constexpr (XF32 && FMT == Q4_K) o.bs = *reinterpret_cast<const f4_t*>(buf + C::ABYTES + C::FBYTES + i * 64 + kq * 16);
                 return o;
             };
@@ -297,20 +300,20 @@ __global__ void __launch_bounds__(64 * WN * WK) __attribute__((amdgpu_waves_per_
                     __builtin_amdgcn_sched_barrier(0);
                 }
             } else {
-                h8_t B[RT], B0[RT];
+                h8_t B[RT], B1[RT];  // (Q6_K: the first and the second scale group's)
                 float s0[RT], s1[RT], p0[RT], p1[RT];
-                f4_t d[RT], e[RT], pd[RT], pe[RT], pfx, pbs;
+                f4_t d[RT], e[RT], pd[RT], pe[RT], pfx[C::GS], pbs;
                 auto add = [&](int t) {  // the previous operand's products into its sums
 #pragma unroll
                     for (int r = 0; r < RT; ++r) {
                         f4_t& ac = acc[r][t];
                         if constexpr (FMT == Q6_K) {
 #pragma unroll
-                            for (int j = 0; j < 4; ++j) ac[j] = fmaf(XF32 ? p1[r] * pfx[j] : p1[r], pe[r][j], ac[j]);
+                            for (int j = 0; j < 4; ++j) ac[j] = fmaf(XF32 ? p1[r] * pfx[C::GS - 1][j] : p1[r], pe[r][j], ac[j]);
                         }
 #pragma unroll
                         for (int j = 0; j < 4; ++j) {
-                            ac[j] = fmaf(XF32 ? p0[r] * pfx[j] : p0[r], pd[r][j], ac[j]);
+                            ac[j] = fmaf(XF32 ? p0[r] * pfx[0][j] : p0[r], pd[r][j], ac[j]);
                             if constexpr (FMT == Q4_K) ac[j] = fmaf(-p1[r], pbs[j], ac[j]);
                         }
                         pin(ac);
@@ -327,9 +330,8 @@ __global__ void __launch_bounds__(64 * WN * WK) __attribute__((amdgpu_waves_per_
                             constexpr int BL = 4 * BPC;  // blocks per load
                             B[r] = direct_operand<FMT>(wd[r][b / BL], b % BL, kq);
                             if constexpr (FMT == Q6_K) {
-                                const uint4 o = __builtin_bit_cast(uint4, B[r]);
-                                const bool g0 = kq < 2;
-                                B0[r] = __builtin_bit_cast(h8_t, make_uint4(g0 ? o.x : 0u, g0 ? o.y : 0u, g0 ? o.z : 0u, g0 ? o.w : 0u));
+                                B1[r] = group_operand(B[r], kq >= 2);
+                                B[r] = group_operand(B[r], kq < 2);
                             }
                             direct_scales<FMT>(cur[r][b / BL], b % BL, 4 * SPL * s + b / BPC < nch, s0[r], s1[r]);
                         }
@@ -342,7 +344,7 @@ __global__ void __launch_bounds__(64 * WN * WK) __attribute__((amdgpu_waves_per_
 #pragma unroll
                     for (int r = 0; r < RT; ++r) {
                         d[r] = product(B[r]);
-                        if constexpr (FMT == Q6_K) e[r] = product(B0[r]);
+                        if constexpr (FMT == Q6_K) e[r] = product(B1[r]);
                     }
                     if (i > 0) add((i - 1) % MT);
 #pragma unroll
@@ -352,7 +354,12 @@ __global__ void __launch_bounds__(64 * WN * WK) __attribute__((amdgpu_waves_per_
                         p0[r] = s0[r];
                         p1[r] = s1[r];
                     }
-                    pfx = cu.fx;
+                    if constexpr (XF32 && C::GS == 2) {  // (two: read with the products, not PA operands ahead: registers)
+                        pfx[0] = power(i, 0);
+                        pfx[1] = power(i, 1);
+                    } else {
+                        pfx[0] = cu.fx;
+                    }
                     pbs = cu.bs;
                 }
                 add(MT - 1);

@@ -36,7 +36,7 @@ static hipError_t launch_tile_one(const MvParams& p, int M, uint32_t x_bytes, hi
 //           Q6_K 14336->4096 at 128 / 512 rows 161 / 642 -> 78.8 / 173
 //           Q8_0 5120x5120 at 64 / 512 rows 41.5 / 341 -> 31.2 / 85.8
 //   fp32 x  Q4_K 4096->14336 at 64 / 512 rows 122 / 439 -> 52.7 / 234
-//           Q6_K 14336->4096 at 64 / 512 rows 112 / 473 -> 93.8 / 325
+//           Q6_K 14336->4096 at 64 / 512 rows 112 / 473 -> 90.2 / 335
 // With few workgroups, several ranges of K per workgroup (x2, x4) make up for the
 // rows they take from it: Q6_K 14336->4096 at 64 rows 175 -> 79.5 (fp16 x).
 struct TileShape {

@@ -81,3 +81,29 @@ def test_direct_f32(gpu, fmt, rt, wk, monkeypatch):
     monkeypatch.setenv("RQMV_DIRECT_WK", wk)
     for n, (rows, cols) in enumerate(shapes(fmt)):
         check(gpu, fmt, rows, cols, "f32", (5, 8, 9, 16, 17, 32, 33, 64, 77), 0 if n else 4)
+
+
+@pytest.mark.parametrize("tile,rt", [("0", "1"), ("0", "2"), ("11", ""), ("22", ""), ("14", "")])
+@pytest.mark.parametrize("big,scale", [(1e5, 0), (1e4, 1)])
+def test_q6_k_f32_groups_of_unlike_scales(gpu, big, scale, tile, rt, monkeypatch):
+    """fp32 activations, one value far above the others in a 16-weight group whose scale
+    is 0 or 1, beside a group of scale about 100: the other group's sum keeps its bits.
+    Each group is a product of its own, scaled on its own, so the limit is the one of
+    ordinary activations (the large value's terms are as large as the whole sum)."""
+    monkeypatch.setenv("RQMV_TILE", tile)
+    monkeypatch.setenv("RQMV_DIRECT_RT", rt)
+    rows, cols = 83, 768
+    w = np.array(synth.weights("q6_k", rows, cols, seed=11)).reshape(-1, 210)
+    w[:, 192:208] = np.random.default_rng(3).integers(90, 120, (len(w), 16))
+    w[:: cols // 256, 192] = scale  # group 0 of every row
+    w = w.reshape(-1)
+    W = gpu.Weight("q6_k", rows, cols, w)
+    for m in (5, 20, 70):
+        x = synth.activations_f32(m * cols, seed=m).reshape(m, cols)
+        x[:, 5] *= big
+        yb = gpu.DeviceBuffer(4 * m * rows)
+        W.matvec(gpu.DeviceBuffer.from_array(x), gpu.DTYPE_F32, m, cols, yb, rows)
+        gpu.synchronize()
+        y = yb.download(np.float32).reshape(m, rows)
+        ref = oracle.matvec_f64("q6_k", w, rows, cols, x, threads=THREADS)
+        assert rel(y, ref) <= limit(cols), (m, rel(y, ref))
