@@ -13,9 +13,11 @@
 //
 // Scales. Q4_K and Q6_K with fp16 activations (FOLD): the weight operand is
 // code x 6-bit scale (Q4_K, an integer of at most 945, exact in fp16) or the
-// two integers code x 16 (scale >> 4) and code x (scale & 15) (Q6_K, in two
-// products), so the matrix cores sum a whole 256-weight block before fp32 arithmetic:
-// the block's d scales the tile once per 256 weights. Q4_K's minimums are one
+// two integers code x 16 (scale / 16) and code x (scale % 16) (Q6_K, in two
+// products; both parts with the scale's sign, so that neither is larger than the
+// scale: -1 as -16 + 15 would take the rounding of sixteen times its sum, 6.6e-7
+// against 8e-8 where every scale is -1), so the matrix cores sum a whole 256-weight
+// block before fp32 arithmetic: the block's d scales the tile once per 256 weights. Q4_K's minimums are one
 // more product per 256 weights, of the eight 6-bit minimums with the eight
 // sub-blocks' activation sums, each sum as three bf16 parts (24 bits).
 // Otherwise every 32-weight block (Q6_K: each 16-weight scale group) is a product
@@ -284,8 +286,9 @@ __global__ void __launch_bounds__(64 * WN * WK) __attribute__((amdgpu_waves_per_
                             } else {
                                 // the scale of this lane's slice: group 2 sub + kq / 2 of the chunk
                                 const uint32_t scw = word(cw.meta, c) >> (16 * sub + 8 * (kq >> 1));
-                                const int sv = (int)(int8_t)(scw & 0xffu);
-                                const _Float16 sh = (_Float16)(float)(sv & ~15), sl = (_Float16)(float)(sv & 15);
+                                const _Float16 sv = (_Float16)(short)(int8_t)(scw & 0xffu);
+                                const _Float16 sh = __builtin_elementwise_trunc(sv * (_Float16)0.0625f) * (_Float16)16.f;
+                                const _Float16 sl = sv - sh;
                                 const h8_t q = direct_operand<FMT>(wd[r][0], b, kq);
                                 B[r] = q * (h8_t){sh, sh, sh, sh, sh, sh, sh, sh};
                                 B2[r] = q * (h8_t){sl, sl, sl, sl, sl, sl, sl, sl};

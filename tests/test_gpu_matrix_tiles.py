@@ -107,3 +107,28 @@ def test_q6_k_f32_groups_of_unlike_scales(gpu, big, scale, tile, rt, monkeypatch
         y = yb.download(np.float32).reshape(m, rows)
         ref = oracle.matvec_f64("q6_k", w, rows, cols, x, threads=THREADS)
         assert rel(y, ref) <= limit(cols), (m, rel(y, ref))
+
+
+@pytest.mark.parametrize("tile", ["11", "12", "15", "14"])
+@pytest.mark.parametrize("scale", [-1, 1, -17])
+def test_q6_k_f16_folded_scales(gpu, tile, scale, monkeypatch):
+    """fp16 activations, every scale of the weight the same small number of either sign.
+    Limit: a 256-weight block is eight accumulations (Q6_K's second product included,
+    sixteen where the scale has both parts), each off by up to 2^-23 of a partial sum
+    that grows with the square root of its length (sum of j / 8, j = 1..8: 4.5), and two
+    fp32 roundings where the blocks are scaled and added."""
+    monkeypatch.setenv("RQMV_TILE", tile)
+    rows, cols = 83, 768
+    w = np.array(synth.weights("q6_k", rows, cols, seed=12)).reshape(-1, 210)
+    w[:, 192:208] = np.int8(scale).view(np.uint8)
+    w = w.reshape(-1)
+    W = gpu.Weight("q6_k", rows, cols, w)
+    bound = 2.0 ** -23 * np.sqrt(4.5 if abs(scale) < 16 else 9.0) + 2.0 ** -23
+    for m in (16, 70):
+        xh, x = activations(m, cols, "f16", seed=m)
+        yb = gpu.DeviceBuffer(4 * m * rows)
+        W.matvec(gpu.DeviceBuffer.from_array(xh), gpu.DTYPE_F16, m, cols, yb, rows)
+        gpu.synchronize()
+        y = yb.download(np.float32).reshape(m, rows)
+        ref = oracle.matvec_f64("q6_k", w, rows, cols, x, threads=THREADS)
+        assert rel(y, ref) <= bound, (m, rel(y, ref), bound)
