@@ -265,6 +265,15 @@ __device__ __forceinline__ void direct_scales(const DirectStep<FMT>& t, int b, b
     }
 }
 
+// Q4_K: a block's activations are summed as 2^-6 of their sum (exactly: a product
+// with this operand), and the minimum multiplies as 2^6 of itself, so that the sum of
+// 32 values of up to fp32's largest does not overflow before a small minimum scales it.
+constexpr float kSumScale = 64.f;
+__device__ __forceinline__ h8_t sum_operand() {
+    constexpr _Float16 u = (_Float16)(1.f / kSumScale);
+    return h8_t{u, u, u, u, u, u, u, u};
+}
+
 constexpr int kDirectMaxWaves = 8;
 
 template <int FMT, int RT, int MT, bool PACK>
@@ -351,6 +360,7 @@ __global__ void __launch_bounds__(64 * kDirectMaxWaves) matvec_mfma_direct(MvPar
                     B[r] = group_operand(B[r], kq < 2);
                 }
                 direct_scales<FMT>(cur[r], b, 4 * s + b / BPC < nch, s0[r], s1[r]);
+                if constexpr (FMT == Q4_K) s1[r] *= kSumScale;
             }
 #pragma unroll
             for (int t = 0; t < MT; ++t) {
@@ -405,9 +415,8 @@ __global__ void __launch_bounds__(64 * kDirectMaxWaves) matvec_mfma_direct(MvPar
                     return D;
                 };
                 f4_t bs = z;
-                if constexpr (FMT == Q4_K) {  // the block's activation sums, unscaled
-                    const h8_t one = {1, 1, 1, 1, 1, 1, 1, 1};
-                    bs = product(one);
+                if constexpr (FMT == Q4_K) {  // the block's activation sums
+                    bs = product(sum_operand());
 #pragma unroll
                     for (int j = 0; j < 4; ++j) bs[j] *= f[j];
                 }

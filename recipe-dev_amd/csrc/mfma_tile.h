@@ -138,8 +138,9 @@ __global__ void __launch_bounds__(64 * WN * WK) __attribute__((amdgpu_waves_per_
         }
     };
     // Sums over a fragment's 32 values per row: with a matrix of ones as the A
-    // operand, the product's every row holds them, the sum of row mn in lane mn.
-    const h8_t ones = {1, 1, 1, 1, 1, 1, 1, 1};
+    // operand, the product's every row holds them, the sum of row mn in lane mn
+    // (fp32 x: times 1 / kSumScale).
+    const h8_t ones = XF32 ? sum_operand() : h8_t{1, 1, 1, 1, 1, 1, 1, 1};
     auto store_x = [&](int win, const Frag (&fr)[FR]) {
         uint8_t* const buf = lds + (win & 1) * C::BUF;
         const f4_t z = {0.f, 0.f, 0.f, 0.f};
@@ -337,6 +338,7 @@ __global__ void __launch_bounds__(64 * WN * WK) __attribute__((amdgpu_waves_per_
                                 B[r] = group_operand(B[r], kq < 2);
                             }
                             direct_scales<FMT>(cur[r][b / BL], b % BL, 4 * SPL * s + b / BPC < nch, s0[r], s1[r]);
+                            if constexpr (FMT == Q4_K) s1[r] *= kSumScale;
                         }
                     }
                     auto product = [&](const h8_t& Wt) {

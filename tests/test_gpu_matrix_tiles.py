@@ -132,3 +132,29 @@ def test_q6_k_f16_folded_scales(gpu, tile, scale, monkeypatch):
         y = yb.download(np.float32).reshape(m, rows)
         ref = oracle.matvec_f64("q6_k", w, rows, cols, x, threads=THREADS)
         assert rel(y, ref) <= bound, (m, rel(y, ref), bound)
+
+
+@pytest.mark.parametrize("fmt", FMTS)
+@pytest.mark.parametrize("tile", ["0", "11", "14"])
+def test_f32_activations_near_the_largest(gpu, fmt, tile, monkeypatch):
+    """fp32 activations of up to 2e38, whose sum over a block overflows fp32, times
+    weights small enough that no output does."""
+    monkeypatch.setenv("RQMV_TILE", tile)
+    rows, cols = 83, 768
+    size, scales = {"q8_0": (34, [0]), "q4_0": (18, [0]), "q4_k": (144, [0, 2]), "q6_k": (210, [208])}[fmt]
+    w = np.array(synth.weights(fmt, rows, cols, seed=13)).reshape(-1, size)
+    for at in scales:
+        d = np.ascontiguousarray(w[:, at:at + 2]).view(np.float16) * np.float16(2.0 ** -8)
+        w[:, at:at + 2] = d.view(np.uint8)
+    w = w.reshape(-1)
+    W = gpu.Weight(fmt, rows, cols, w)
+    for m in (5, 20, 70):
+        x = (synth.activations_f32(m * cols, seed=m) * np.float32(5e37)).reshape(m, cols)
+        x[:, :32] = np.abs(x[:, :32])
+        yb = gpu.DeviceBuffer(4 * m * rows)
+        W.matvec(gpu.DeviceBuffer.from_array(x), gpu.DTYPE_F32, m, cols, yb, rows)
+        gpu.synchronize()
+        y = yb.download(np.float32).reshape(m, rows)
+        ref = oracle.matvec_f64(fmt, w, rows, cols, x, threads=THREADS)
+        assert np.abs(ref).max() < 3e38 and np.isfinite(y).all(), (fmt, m)
+        assert rel(y, ref) <= limit(cols), (fmt, m)
