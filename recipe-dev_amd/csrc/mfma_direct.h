@@ -28,7 +28,7 @@
 // trips of a wave's two or four steps; the weights' bytes take a fifth of the
 // time. Measured against the staged form this replaces (kernel us, fp32 x): Q4_K
 // 4096x4096 at 5 rows 83.8 -> 12.2 (780 GB/s), Q6_K 14336->4096 at 77 rows
-// 3363 -> 114 (79 TFLOP/s).
+// 3363 -> 106 (85 TFLOP/s).
 #pragma once
 
 #include <hip/hip_ext.h>
@@ -85,16 +85,16 @@ __device__ __forceinline__ float max_over_pair(float v) {
     swap_bit4(a, b);
     return fmaxf(__builtin_bit_cast(float, a), __builtin_bit_cast(float, b));
 }
-// Both pairs' largest, in all four lanes.
-__device__ __forceinline__ void pair_maxima(float v, float& first, float& second) {
-    uint32_t a = __builtin_bit_cast(uint32_t, max_over_pair(v)), b = opaque(a);
+// A value of each pair, first and second, in all four lanes.
+__device__ __forceinline__ void both_pairs(float v, float& first, float& second) {
+    uint32_t a = __builtin_bit_cast(uint32_t, v), b = opaque(a);
     swap_bit5(a, b);
     first = __builtin_bit_cast(float, a);
     second = __builtin_bit_cast(float, b);
 }
 __device__ __forceinline__ float max_over_slices(float v) {
     float a, b;
-    pair_maxima(v, a, b);
+    both_pairs(max_over_pair(v), a, b);
     return fmaxf(a, b);
 }
 
@@ -107,6 +107,16 @@ __device__ __forceinline__ float rotate_to_rows(float v) {
     r = __builtin_amdgcn_update_dpp(r, s, 0x128, 0x4, 0xF, false);  // row 2: row_ror:8
     r = __builtin_amdgcn_update_dpp(r, s, 0x124, 0x8, 0xF, false);  // row 3: row_ror:4
     return __builtin_bit_cast(float, r);
+}
+// The same of a value that rows 0 and 1, and rows 2 and 3, hold alike, for each pair's
+// (rows 1 and 3 turn by 12 before the exchange, rows 2 and 3 by 8 after it).
+__device__ __forceinline__ void rotate_pairs_to_rows(float v, float& first, float& second) {
+    const int s = __builtin_bit_cast(int, v);
+    v = __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(s, s, 0x12C, 0xA, 0xF, false));  // row_ror:12
+    both_pairs(v, first, second);
+    const int a = __builtin_bit_cast(int, first), b = __builtin_bit_cast(int, second);
+    first = __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(a, a, 0x128, 0xC, 0xF, false));  // row_ror:8
+    second = __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(b, b, 0x128, 0xC, 0xF, false));
 }
 template <int J>
 __device__ __forceinline__ float row_bcast(float v) {
@@ -380,24 +390,21 @@ __global__ void __launch_bounds__(64 * kDirectMaxWaves) matvec_mfma_direct(MvPar
                 for (int e = 0; e < 8; ++e) am = fmaxf(am, fabsf(v[e]));
                 uint32_t hi[4], lo[4];
                 float f[4], g[4];  // the inverse powers of rows 4 kq + j (g: the second group's)
-                auto rows_of = [](int k, float (&o)[4]) {
-                    const float fx = rotate_to_rows(pow2f(-k));
+                auto rows_of = [](float fx, float (&o)[4]) {
                     o[0] = row_bcast<0>(fx);
                     o[1] = row_bcast<1>(fx);
                     o[2] = row_bcast<2>(fx);
                     o[3] = row_bcast<3>(fx);
                 };
+                const int ks = block_shift(FMT == Q6_K ? max_over_pair(am) : max_over_slices(am));
+                split_hi_lo(v, pow2f(ks), hi, lo);
                 if constexpr (FMT == Q6_K) {
-                    float am0, am1;
-                    pair_maxima(am, am0, am1);
-                    const int k0 = block_shift(am0), k1 = block_shift(am1);
-                    split_hi_lo(v, pow2f(kq < 2 ? k0 : k1), hi, lo);
-                    rows_of(k0, f);
-                    rows_of(k1, g);
+                    float f0, f1;
+                    rotate_pairs_to_rows(pow2f(-ks), f0, f1);
+                    rows_of(f0, f);
+                    rows_of(f1, g);
                 } else {
-                    const int ks = block_shift(max_over_slices(am));
-                    split_hi_lo(v, pow2f(ks), hi, lo);
-                    rows_of(ks, f);
+                    rows_of(rotate_to_rows(pow2f(-ks)), f);
                 }
                 h8_t A[2];
                 if constexpr (PACK) {

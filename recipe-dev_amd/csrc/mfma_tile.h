@@ -84,6 +84,7 @@ __global__ void __launch_bounds__(64 * WN * WK) __attribute__((amdgpu_waves_per_
     constexpr int DW = RT == 1 && !LEAN ? 3 : 2;          // steps of weights in rotation (DW - 1 in flight)
     constexpr int XD = LEAN || (C::FOLD && RT * MT >= 16) ? 1 : 2;  // windows of activations in flight (one: registers)
     constexpr int PA = LEAN ? (XF32 ? 1 : 3) : XF32 ? 2 : RT * MT >= 16 ? 3 : 6;  // operands read from LDS ahead
+    constexpr bool FXA = C::GS == 1 || (!LEAN && RT == 1);  // fp32 x: powers read ahead with the operands (Q6_K's two: registers)
     static_assert(WB * MT % WN == 0 && WPS == 2, "fragments divide over the waves; two windows a step");
     constexpr bool FOLD = C::FOLD;
     extern __shared__ uint4 smem[];
@@ -249,14 +250,17 @@ __global__ void __launch_bounds__(64 * WN * WK) __attribute__((amdgpu_waves_per_
             // and holds all of them in registers).
             struct Operand {
                 h8_t a[C::XN];
-                f4_t fx, bs;
+                f4_t fx[FXA ? C::GS : 1], bs;
             };
             auto power = [&](int i, int h) { return *reinterpret_cast<const f4_t*>(buf + C::ABYTES + (i * C::GS + h) * 64 + kq * 16); };
             auto read = [&](int i) {
                 Operand o;
 #pragma unroll
                 for (int h = 0; h < C::XN; ++h) o.a[h] = *reinterpret_cast<const h8_t*>(buf + (i * C::XN + h) * 1024 + lane * 16);
-                if constexpr (XF32 && C::GS == 1) o.fx = power(i, 0);
+                if constexpr (XF32 && FXA) {
+#pragma unroll
+                    for (int h = 0; h < C::GS; ++h) o.fx[h] = power(i, h);
+                }
                 if constexpr (XF32 && FMT == Q4_K) o.bs = *reinterpret_cast<const f4_t*>(buf + C::ABYTES + C::FBYTES + i * 64 + kq * 16);
                 return o;
             };
@@ -359,12 +363,8 @@ __global__ void __launch_bounds__(64 * WN * WK) __attribute__((amdgpu_waves_per_
                         p0[r] = s0[r];
                         p1[r] = s1[r];
                     }
-                    if constexpr (XF32 && C::GS == 2) {  // (two: read with the products, not PA operands ahead: registers)
-                        pfx[0] = power(i, 0);
-                        pfx[1] = power(i, 1);
-                    } else {
-                        pfx[0] = cu.fx;
-                    }
+#pragma unroll
+                    for (int h = 0; h < C::GS; ++h) pfx[h] = XF32 && !FXA ? power(i, h) : cu.fx[FXA ? h : 0];
                     pbs = cu.bs;
                 }
                 add(MT - 1);
