@@ -95,6 +95,10 @@ hipError_t launch_matvec_mfma(int fmt, int M, const MvParams& p, int cus, hipStr
 // activations span less than 4 GiB.
 hipError_t launch_matvec_f32(int fmt, const MvParams& p, int M, int cus, hipStream_t stream, hipEvent_t ev0 = nullptr,
                              hipEvent_t ev1 = nullptr);
+// Estimated times (us) of the direct form (more than 16 rows) and of fp16 activations
+// in launches of 32 rows, which the tiled form's plan is compared with.
+float direct_us(int fmt, int M, int64_t rows, int64_t cols, int cus);
+float stream_us(int fmt, int M, int64_t rows, int64_t cols, int cus);
 // The tiled form (mfma_tile.hip), for many activation rows. tile_takes: whether
 // a product of M rows runs in it rather than in the streaming form (fp16) or the
 // direct one (fp32).

@@ -174,6 +174,31 @@ static hipError_t launch_mfma_fmt(int W, const MvParams& p, int M, uint32_t x_by
     return launch_mfma_w<FMT, 1>(W, p, M, x_bytes, stream, ev0, ev1);
 }
 
+// Estimated time (us) of a product in launches of 32 rows, for the choice between
+// them and the tiled form above 32 rows: per launch 5 us and, per step of 256 values,
+// what the row tiles cost that one wave or two take (up to one row tile per CU, up to
+// two, and above by their count), or on long rows of few row tiles, where four waves
+// split K, `split` for each two of a CU's. A last launch of 16 rows or fewer takes two
+// thirds on long rows (the split-K form). Fitted to 1,133 products of 33 to 160 rows
+// (within 14 % of the estimates, root mean square).
+float stream_us(int fmt, int M, int64_t rows, int64_t cols, int cus) {
+    struct Cost {
+        float one, two, more, split;
+    };
+    const Cost c = fmt == Q4_0   ? Cost{0.37f, 0.56f, 1.42e-3f, 0.33f}
+                   : fmt == Q4_K ? Cost{0.48f, 0.78f, 1.90e-3f, 0.37f}
+                   : fmt == Q8_0 ? Cost{0.70f, 0.82f, 1.70e-3f, 0.36f}
+                                 : Cost{0.63f, 1.02f, 2.13e-3f, 0.48f};
+    const int64_t tiles = (rows + 15) / 16;
+    const float steps = (float)((cols + 255) / 256);
+    float each = tiles <= cus ? c.one : c.two;
+    if (c.more * (float)tiles > each) each = c.more * (float)tiles;
+    if (cols > 8192 && tiles < cus) each = c.split * (float)((2 * tiles + cus - 1) / cus);
+    const int rest = M % 32;
+    const float launches = (float)(M / 32) + (rest == 0 ? 0.f : rest <= 16 && cols > 8192 ? 0.65f : 1.f);
+    return launches * (5.f + steps * each);
+}
+
 hipError_t launch_matvec_mfma(int fmt, int M, const MvParams& p, int cus, hipStream_t stream,
                               hipEvent_t ev0, hipEvent_t ev1) {
     if (M < 1 || M > 32) return hipErrorInvalidValue;

@@ -26,45 +26,54 @@ static hipError_t launch_tile_one(const MvParams& p, int M, uint32_t x_bytes, hi
     return hipGetLastError();
 }
 
-// The shapes, and what a step of 256 values of K takes a workgroup in each (us,
-// measured with one workgroup per CU at most, less a launch's 4 us): the plan takes
-// the shape whose steps, times the rounds of workgroups over the chip, are fewest.
-// Kernel us at the shape the plan takes, against the streaming form in launches of
+// The shapes, and what a step of 256 values of K and a round of workgroups over the
+// chip take in each (us; 0: not built, since its registers spill and no product was
+// fastest in it). Fitted to 3,847 products of 256 to 25,600 rows, 1,024 to 14,336
+// columns and 17 to 512 activation rows, each timed in every shape (within 5 to 9 % of
+// the estimates, root mean square). The plan takes the shape whose rounds cost the
+// fewest; over the same products its choice, this form or the other, takes 0.4 % more
+// than the best of all on average, 20 % at most.
+// us a product at the shape the plan takes, against the streaming form in launches of
 // 32 rows (fp16 x) or the direct form (fp32 x):
-//   fp16 x  Q4_K 4096->14336 at 64 / 512 rows 50.6 / 393 -> 29.2 / 114 (528 TFLOP/s)
-//           Q4_0 4096->14336 at 512 rows -> 97.4 (617 TFLOP/s)
-//           Q6_K 14336->4096 at 128 / 512 rows 161 / 642 -> 78.8 / 173
-//           Q8_0 5120x5120 at 64 / 512 rows 41.5 / 341 -> 31.2 / 85.8
-//   fp32 x  Q4_K 4096->14336 at 64 / 512 rows 122 / 439 -> 52.7 / 234
-//           Q6_K 14336->4096 at 64 / 512 rows 112 / 473 -> 90.2 / 335
+//   fp16 x  Q4_K 4096->14336 at 64 / 512 rows 48.5 / 381 -> 28.5 / 108 (557 TFLOP/s)
+//           Q4_0 4096->14336 at 512 rows 332 -> 96.3 (624 TFLOP/s)
+//           Q6_K 14336->4096 at 128 / 512 rows 157 / 608 -> 82 / 161
+//           Q8_0 5120x5120 at 64 / 512 rows 41.5 / 341 -> 30.3 / 82.1
+//   fp32 x  Q4_K 4096->14336 at 64 / 512 rows 79 / 498 -> 48 / 242
+//           Q6_K 14336->4096 at 512 rows 589 -> 323
 // With few workgroups, several ranges of K per workgroup (x2, x4) make up for the
-// rows they take from it: Q6_K 14336->4096 at 64 rows 175 -> 79.5 (fp16 x).
+// rows they take from it: Q6_K 14336->4096 at 64 rows 159 -> 79 (fp16 x).
 struct TileShape {
     int id, rt, mt, wn, wk;  // mt for fp16 x, half of it for fp32 x
     float step[2][4];        // us per step: [fp32 x][Q4_0, Q4_K, Q8_0, Q6_K]
+    float round;             // us per round
 };
 constexpr TileShape kTileShapes[] = {
-    {11, 1, 4, 8, 1, {{2.15f, 2.2f, 2.8f, 3.0f}, {2.75f, 2.7f, 3.25f, 3.7f}}},
-    {12, 1, 8, 8, 1, {{3.0f, 3.05f, 3.5f, 3.9f}, {3.9f, 4.5f, 4.55f, 5.4f}}},
-    {22, 2, 8, 8, 1, {{5.8f, 6.8f, 6.9f, 9.5f}, {5.9f, 7.0f, 6.9f, 10.5f}}},
-    {15, 1, 4, 4, 2, {{2.9f, 3.0f, 3.4f, 3.6f}, {3.5f, 3.8f, 4.15f, 4.45f}}},
-    {14, 1, 4, 2, 4, {{4.7f, 5.2f, 5.4f, 5.4f}, {5.8f, 6.6f, 5.6f, 6.5f}}},
+    {11, 1, 4, 8, 1, {{2.02f, 2.06f, 2.51f, 2.70f}, {2.38f, 2.72f, 2.89f, 3.60f}}, 0.6f},
+    {12, 1, 8, 8, 1, {{3.06f, 3.08f, 3.44f, 3.82f}, {3.62f, 4.41f, 4.09f, 5.36f}}, 2.8f},
+    {22, 2, 8, 8, 1, {{5.26f, 5.81f, 6.02f, 0.00f}, {5.60f, 6.93f, 6.45f, 10.87f}}, 2.6f},
+    {15, 1, 4, 4, 2, {{2.49f, 2.78f, 2.98f, 3.28f}, {3.07f, 3.52f, 3.52f, 4.17f}}, 2.5f},
+    {14, 1, 4, 2, 4, {{3.73f, 4.33f, 4.21f, 4.60f}, {4.70f, 5.34f, 5.18f, 5.74f}}, 3.1f},
 };
 
 static int fmt_slot(int fmt) { return fmt == Q4_0 ? 0 : fmt == Q4_K ? 1 : fmt == Q8_0 ? 2 : 3; }
 
-// The best shape for a product and its estimated time (us). Shape 11's workgroups run
-// two to a CU, where a round of them takes 0.82 of two. RQMV_TILE names a shape instead.
+// The best shape for a product and its estimated time (us). Rounds are those of the XCD
+// with the most workgroups (an XCD takes every eighth tile of rows). Of several, each
+// takes 1.04 of one alone, in shape 11, whose workgroups run two to a CU, 0.9 (fp16 x) or
+// 0.82. RQMV_TILE names a shape instead.
 static const TileShape& tile_plan(int fmt, bool f32, int64_t M, int64_t rows, int64_t cols, int cus, float* us) {
     const char* env = getenv("RQMV_TILE");
     const int want = env && *env ? atoi(env) : 0;
     const TileShape* best = nullptr;
     for (const TileShape& s : kTileShapes) {
+        const float step = s.step[f32][fmt_slot(fmt)];
+        if (step == 0.f) continue;
         const int64_t bn = 16 * s.rt * s.wn, bm = 16 * (f32 ? s.mt / 2 : s.mt);
-        const int64_t wgs = (rows + bn - 1) / bn * ((M + bm - 1) / bm);
+        const int64_t wgs = ((rows + bn - 1) / bn + 7) / 8 * 8 * ((M + bm - 1) / bm);
         const int64_t steps = ((cols + 255) / 256 + s.wk - 1) / s.wk, rounds = (wgs + cus - 1) / cus;
-        const float share = s.id == 11 && rounds > 1 ? 0.82f : 1.f;
-        const float t = 4.f + s.step[f32][fmt_slot(fmt)] * (float)steps * (float)rounds * share;
+        const float each = rounds == 1 ? 1.f : s.id != 11 ? 1.04f : f32 ? 0.82f : 0.9f;
+        const float t = 1.5f + (float)rounds * each * (step * (float)steps + s.round);
         if (s.id == want || (!best || (t < *us && best->id != want))) {
             best = &s;
             *us = t;
@@ -81,38 +90,27 @@ static hipError_t launch_tile_fmt(int shape, const MvParams& p, int M, uint32_t 
     switch (shape) {
         case 11: return RQ_SHAPE(1, S, 8, 1);
         case 12: return RQ_SHAPE(1, L, 8, 1);
-        case 22: return RQ_SHAPE(2, L, 8, 1);
+        case 22:
+            if constexpr (FMT == Q6_K && !XF32) return hipErrorInvalidValue;  // (not built: the plan never names it)
+            else return RQ_SHAPE(2, L, 8, 1);
         case 15: return RQ_SHAPE(1, S, 4, 2);
         default: return RQ_SHAPE(1, S, 2, 4);
     }
 #undef RQ_SHAPE
 }
 
-// Against the other forms, by the same measure. The streaming form (fp16 x) takes 32
-// rows a launch and per launch 3 us and the larger of 0.65 us (Q8_0 0.9) a step of 256
-// values and 1.6 ns a step and row tile (Q4_K 4096->14336 25 us, Q8_0 5120x5120 21,
-// Q6_K 5120->25600 55); up to 32 rows it is always ahead (Q4_K 4096x4096 at 20 rows 13.9
-// against 19.2). The direct form (fp32 x) is ahead up to 16 rows; above, it takes the
-// larger of 0.9 us a step and 3.6 ns a step and row tile (2.5 with two row tiles per
-// wave) for one or two activation tiles per wave, and where the rows fall into groups
-// of three tiles 3.5 ns a group (Q6_K 14336->4096 at 77 rows 106 against 120); otherwise
-// it is behind. RQMV_TILE=0 keeps every product off the tiled form.
+// Against the other form, by the same measure (stream_us, direct_us). The streaming
+// form (fp16 x) is always ahead up to 32 rows (Q4_K 4096x4096 at 20 rows 13.9 against
+// 19.2), the direct form (fp32 x) up to 16. RQMV_TILE=0 keeps every product off the
+// tiled form.
 bool tile_takes(int fmt, int xtype, int M, int64_t rows, int64_t cols, int cus) {
     const char* env = getenv("RQMV_TILE");
     if (env && *env) return *env != '0';
-    float us = 0.f;
     const bool f32 = xtype == X_F32;
     if (M <= 16 || (!f32 && M <= 32)) return false;
+    float us = 0.f;
     tile_plan(fmt, f32, M, rows, cols, cus, &us);
-    const float steps = (float)((cols + 255) / 256), units = steps * (float)((rows + 15) / 16);
-    if (f32) {
-        const int tiles = (M + 15) / 16, groups = (tiles + 3) / 4;
-        if (M > 32 && (groups == 1 || (tiles + groups - 1) / groups != 3)) return true;
-        const float b = (M > 32 ? 3.5e-3f * (float)groups : (rows + 15) / 16 > cus ? 2.5e-3f : 3.6e-3f) * units;
-        return us < 4.f + (0.9f * steps > b ? 0.9f * steps : b);
-    }
-    const float a = (fmt == Q8_0 ? 0.9f : 0.65f) * steps, b = 1.6e-3f * units;
-    return us < (float)((M + 31) / 32) * (3.f + (a > b ? a : b));
+    return us < (f32 ? direct_us(fmt, M, rows, cols, cus) : stream_us(fmt, M, rows, cols, cus));
 }
 
 hipError_t launch_matvec_tile(int fmt, int xtype, int M, const MvParams& p, int cus, hipStream_t stream, hipEvent_t ev0,

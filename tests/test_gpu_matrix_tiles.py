@@ -1,6 +1,6 @@
 """The matrix-core forms for fp32 activations and for many activation rows, at
 the edges of their tiles: the direct form with one and two row tiles per wave,
-the packed operand (up to eight rows) and one to four 16-row tiles; the tiled
+the packed operand (up to eight rows) and one to three 16-row tiles; the tiled
 form in each of its workgroup shapes, fp16 and fp32 activations. Partial tiles,
 ranges of K with and without steps, rows whose last step or block is partial and
 rows of more than one 64-chunk group, strided rows of x and y, one value far
@@ -74,13 +74,23 @@ def test_tiled(gpu, fmt, shape, xdt, monkeypatch):
 
 
 @pytest.mark.parametrize("fmt", FMTS)
-@pytest.mark.parametrize("rt,wk", [("1", "8"), ("2", "4"), ("2", "1")])
+@pytest.mark.parametrize("rt,wk", [("1", "8"), ("2", "8"), ("2", "4"), ("2", "1")])
 def test_direct_f32(gpu, fmt, rt, wk, monkeypatch):
     monkeypatch.setenv("RQMV_TILE", "0")
     monkeypatch.setenv("RQMV_DIRECT_RT", rt)
     monkeypatch.setenv("RQMV_DIRECT_WK", wk)
     for n, (rows, cols) in enumerate(shapes(fmt)):
         check(gpu, fmt, rows, cols, "f32", (5, 8, 9, 16, 17, 32, 33, 64, 77), 0 if n else 4)
+
+
+@pytest.mark.parametrize("fmt", FMTS)
+@pytest.mark.parametrize("xdt", ["f16", "f32"])
+def test_as_planned(gpu, fmt, xdt):
+    """The form and shape the plan takes, on both sides of its lines: few and many row
+    tiles, short and long rows, 16-row groups that fall by ones, twos and threes."""
+    short, longer = (512, 8448) if fmt in ("q4_k", "q6_k") else (480, 8416)
+    for rows, cols in ((40, short), (4200, short), (40, longer)):
+        check(gpu, fmt, rows, cols, xdt, (17, 33, 48, 65, 112, 145), 0)
 
 
 @pytest.mark.parametrize("tile,rt", [("0", "1"), ("0", "2"), ("11", ""), ("22", ""), ("14", "")])
