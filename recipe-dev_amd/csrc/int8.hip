@@ -455,7 +455,7 @@ __global__ __launch_bounds__(kI8Threads) void int8_slices_kernel(I8Launch p) {
 // each wave reads and unpacks its two weight rows once for all of them. Every output sees
 // the operations of the one-row kernel in their order. Step 32, us at 4 / 8 rows with a
 // workgroup per activation row -> four rows a workgroup: Q4_K 4096->14336 27.7 / 52.5 ->
-// 22.9 / 37.8, Q6_K 33.5 / 62.0 -> 22.6 / 35.9, Q4_0 33.2 / 61.6 -> 24.4 / 35.5; Q8_0
+// 22.3 / 36.2, Q6_K 33.5 / 62.0 -> 21.2 / 32.3, Q4_0 33.2 / 61.6 -> 24.4 / 35.5; Q8_0
 // 5120x5120 14.3 / 25.9 -> 13.1 (two rows) / 20.5. Bound by the records' LDS reads and
 // the sums' round trip.
 template <int MR>
@@ -784,25 +784,51 @@ size_t int8_lds_bytes(int64_t cols) {
     return (size_t)cols + ((tail + 3) & ~size_t(3)) * 4 + (size_t)(kI8Threads / 64) * 2048;
 }
 
-// Activation rows per workgroup of a batch: four from four rows and two from two, where
-// that leaves two workgroups per CU (Q8_0 5120x5120 at four rows 14.3 us alone, 13.1 by
-// twos, 15.9 by fours; Q4_K 1111x2048 at four 6.6 / 6.5 / 8.3) and their records and the
-// waves' buffers fit 64 KiB of LDS. Three and five rows would leave a third of the places
-// empty, and run alone. RQMV_I8_ROWS=1/2/4 overrides it for tuning.
-static int int8_rows(int M, int64_t rows, int K, size_t (*wave_bytes)(int)) {
-    const int64_t tiles = (rows + kI8Rows - 1) / kI8Rows;
+// Activation rows per workgroup of a batch: one, two or four, whichever costs least. A
+// CU's workgroups (two at least: fewer take as long) cost w of a one-row workgroup's time
+// each, w as measured on batches of 15 rows and more (us, one / two / four rows a
+// workgroup, step 32: Q4_K 4096->14336 at 64 rows 378 / 358 / 264, Q6_K 548 / 415 / 295;
+// four cost more on longer rows, whose records leave room for fewer workgroups). One-row
+// workgroups of Q8_0 wait for memory once the weight outgrows the eight L2s of 4 MB (486 /
+// 310 / 220). Last groups may have places empty: Q6_K 25600x1024 at three rows 39.9 / 39.9 /
+// 28.9, Q8_0 14336x4096 at five 37.8 / 31.1 / 30.2. Over 4,088 batches the choice takes
+// 0.7 % more than the best of the three on average and is behind one row a workgroup by
+// more than 3 % in 61 (12 % at most). The records and the waves' buffers stay within 64 KiB
+// of LDS. RQMV_I8_ROWS=1/2/4 overrides it for tuning.
+static int int8_rows(int fmt, int step, int M, int64_t rows, int K, size_t weight_bytes, int cus, size_t (*wave_bytes)(int)) {
+    auto fits = [&](int mr) { return (size_t)mr * i8_row_bytes(K) + (size_t)(kI8Threads / 64) * wave_bytes(mr) <= 65536; };
     int mr = 1;
-    if (M >= 2 && M != 3 && M != 5) mr = M >= 4 && tiles * ((M + 3) / 4) >= 512 ? 4 : tiles * ((M + 1) / 2) >= 512 ? 2 : 1;
     const char* env = getenv("RQMV_I8_ROWS");
-    if (env && *env) mr = atoi(env) >= 4 ? 4 : atoi(env) >= 2 ? 2 : 1;
-    while (mr > 1 && (size_t)mr * i8_row_bytes(K) + (size_t)(kI8Threads / 64) * wave_bytes(mr) > 65536) mr >>= 1;
+    if (env && *env) {
+        mr = atoi(env) >= 4 ? 4 : atoi(env) >= 2 ? 2 : 1;
+        while (mr > 1 && !fits(mr)) mr >>= 1;
+        return mr;
+    }
+    const bool s32 = step == 32;
+    float two = 0.f, four = 0.f;
+    switch (fmt) {
+        case Q4_0: two = s32 ? 1.92f : 1.90f, four = s32 ? 3.00f : 3.10f; break;
+        case Q4_K: two = s32 ? 1.85f : 1.50f, four = s32 ? 2.70f : 2.75f; break;
+        case Q8_0: two = s32 ? 1.65f : 1.70f, four = s32 ? 2.75f : 3.00f; break;
+        default: two = s32 ? 1.52f : 1.62f, four = s32 ? 2.15f : 2.70f; break;
+    }
+    if (fmt == Q8_0 && weight_bytes > (24u << 20)) two *= 0.77f, four *= 0.69f;
+    four *= 1.f + 0.1f * ((float)K / 4096.f - 1.f);
+    const int64_t tiles = (rows + kI8Rows - 1) / kI8Rows;
+    auto cost = [&](int n, float w) {
+        const int64_t per_cu = (tiles * ((M + n - 1) / n) + cus - 1) / cus;
+        return w * (float)(per_cu > 2 ? per_cu : 2);
+    };
+    float best = cost(1, 1.f);
+    if (M >= 2 && fits(2) && cost(2, two) < best) mr = 2, best = cost(2, two);
+    if (M >= 3 && fits(4) && cost(4, four) < best) mr = 4;
     return mr;
 }
 
 template <int FMT>
-static hipError_t launch_blocks(const I8Launch& p, hipStream_t stream) {
+static hipError_t launch_blocks(const I8Launch& p, int cus, hipStream_t stream) {
     auto wave_bytes = [](int mr) -> size_t { return block_wave_bytes<FMT>(mr); };
-    const int mr = int8_rows(p.M, p.rows, p.K, wave_bytes);
+    const int mr = int8_rows(FMT, 256, p.M, p.rows, p.K, p.P.bytes, cus, wave_bytes);
     const dim3 grid((unsigned)((p.rows + kI8Rows - 1) / kI8Rows), (unsigned)((p.M + mr - 1) / mr));
     size_t lds = int8_lds_bytes(p.K);
     void (*kernel)(I8Launch) = FMT == Q4_K ? int8_q4k256_kernel : int8_q6k256_kernel;
@@ -815,8 +841,8 @@ static hipError_t launch_blocks(const I8Launch& p, hipStream_t stream) {
 }
 
 template <int FMT>
-static hipError_t launch_slices(const I8Launch& p, hipStream_t stream) {
-    const int mr = int8_rows(p.M, p.rows, p.K, [](int) -> size_t { return 2048; });
+static hipError_t launch_slices(const I8Launch& p, int cus, hipStream_t stream) {
+    const int mr = int8_rows(FMT, p.step, p.M, p.rows, p.K, p.P.bytes, cus, [](int) -> size_t { return 2048; });
     const dim3 grid((unsigned)((p.rows + kI8Rows - 1) / kI8Rows), (unsigned)((p.M + mr - 1) / mr));
     size_t lds = int8_lds_bytes(p.K);
     auto kernel = int8_slices_kernel<FMT>;
@@ -829,15 +855,15 @@ static hipError_t launch_slices(const I8Launch& p, hipStream_t stream) {
 }
 
 hipError_t launch_matvec_int8(int fmt, const Planes& P, int64_t rows, int K, const float* x, int M, int64_t ldx,
-                              float* y, int64_t ldy, int step, int tail, hipStream_t stream) {
+                              float* y, int64_t ldy, int step, int tail, int cus, hipStream_t stream) {
     I8Launch p{P, rows, K, x, ldx, y, ldy, M, step, tail};
-    if (step == 256 && fmt == Q4_K) return launch_blocks<Q4_K>(p, stream);
-    if (step == 256 && fmt == Q6_K) return launch_blocks<Q6_K>(p, stream);
+    if (step == 256 && fmt == Q4_K) return launch_blocks<Q4_K>(p, cus, stream);
+    if (step == 256 && fmt == Q6_K) return launch_blocks<Q6_K>(p, cus, stream);
     switch (fmt) {
-        case Q4_K: return launch_slices<Q4_K>(p, stream);
-        case Q6_K: return launch_slices<Q6_K>(p, stream);
-        case Q8_0: return launch_slices<Q8_0>(p, stream);
-        case Q4_0: return launch_slices<Q4_0>(p, stream);
+        case Q4_K: return launch_slices<Q4_K>(p, cus, stream);
+        case Q6_K: return launch_slices<Q6_K>(p, cus, stream);
+        case Q8_0: return launch_slices<Q8_0>(p, cus, stream);
+        case Q4_0: return launch_slices<Q4_0>(p, cus, stream);
         default: return hipErrorInvalidValue;
     }
 }

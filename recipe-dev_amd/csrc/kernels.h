@@ -112,7 +112,7 @@ size_t mfma_lds_bytes(int fmt, int M, int64_t rows, int cus);
 // n < rows, m < M; tail: the last position folds 256-step Q4_K blocks whole.
 size_t int8_lds_bytes(int64_t cols);
 hipError_t launch_matvec_int8(int fmt, const Planes& P, int64_t rows, int K, const float* x, int M, int64_t ldx,
-                              float* y, int64_t ldy, int step, int tail, hipStream_t stream);
+                              float* y, int64_t ldy, int step, int tail, int cus, hipStream_t stream);
 hipError_t launch_q8_records(const float* x, int K, int step, float* d, int8_t* codes, hipStream_t stream);
 
 }  // namespace rq

@@ -780,7 +780,7 @@ int rqmv_matvec_int8(const rqmv_weight* w, const float* x_dev, int m, int64_t ld
         return fail(RQMV_EINVAL, "int8: x must be 16-byte aligned and ldx a multiple of 4");
     if (rq::int8_lds_bytes(w->cols) > info.lds_limit) return fail(RQMV_EINVAL, "int8: cols too large for the LDS records");
     hipError_t e = rq::launch_matvec_int8(w->fmt, planes_of(w, 0), rows, (int)w->cols, x_dev, m, ldx, y_dev, ldy, step,
-                                          (flags & RQMV_INT8_TAIL) ? 1 : 0, static_cast<hipStream_t>(stream));
+                                          (flags & RQMV_INT8_TAIL) ? 1 : 0, info.cus, static_cast<hipStream_t>(stream));
     return e == hipSuccess ? RQMV_OK : hip_fail(e, "int8 launch");
 }
 

@@ -187,3 +187,16 @@ def test_batches_by_rows_per_workgroup(gpu, mr, step, fmt, monkeypatch):
         x = np.stack([synth.activations_f32(cols, seed=50 + i) for i in range(m)])
         W = gpu.Weight(fmt, rows, cols, w)
         assert _bits_equal(gpu.contract_int8(W, x, step), oracle.int8_matvec(fmt, w, rows, cols, x, step)), (rows, cols, m)
+
+
+@pytest.mark.parametrize("fmt", ["q4_k", "q6_k", "q4_0", "q8_0"])
+@pytest.mark.parametrize("step", [32, 256])
+def test_batches_as_planned(gpu, step, fmt):
+    """Batches with the rows per workgroup that the plan takes for them: counts that fill
+    the last workgroup and counts that leave places empty, few row tiles and many."""
+    for rows, cols in ((4112, 512), (35, 2048)):
+        w = synth.weights(fmt, rows, cols, seed=rows)
+        x = np.stack([synth.activations_f32(cols, seed=70 + i) for i in range(13)])
+        W = gpu.Weight(fmt, rows, cols, w)
+        for m in (2, 3, 5, 6, 13):
+            assert _bits_equal(gpu.contract_int8(W, x[:m], step), oracle.int8_matvec(fmt, w, rows, cols, x[:m], step)), (rows, m)
