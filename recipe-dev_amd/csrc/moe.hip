@@ -25,7 +25,7 @@
 namespace rq {
 
 constexpr int kMoeThreads = 256;  // workgroup size of the MoE kernels (four waves)
-constexpr int kMoeBatchMin = 16;  // positions from which the products take their batch forms
+constexpr int kMoeBatchMin = 16;  // positions from which the products may take their batch forms
 constexpr int kMoeOwnRouteMax = 2;  // positions per launch up to which every wave routes on its own
 
 static size_t al(size_t v) { return (v + 255) & ~size_t(255); }
@@ -950,9 +950,15 @@ static hipError_t down_fmt(const MoeDims& d, const MoeBank& down, const MoeBank&
     // 1422 in the form below against 49.5 / 67.4 / 159.0 / 1027 (64, 64, 128, 128 rows;
     // 32 rows 51.0 / 68.8 / 171.5 / 1105). Its weights are read with ordinary loads: with
     // the non-temporal ones of the one-position form, which mark lines for early
-    // eviction, the same steps took 50 / 74.6 / 174.8 / 1223.
+    // eviction, the same steps took 50 / 74.6 / 174.8 / 1223. The encoding costs a launch
+    // and the blocks fewer rows per staged position, so small products stay with the form
+    // below: us a step at 16 positions, Q6_K 512x(8 slots of 512) 33.3 against 44.6, Q4_0
+    // 1024x(2 of 768) 22.5 against 25.5, but Q8_0 2048x(6 of 512) 70.3 against 62.1. Over 560 batches of 16 to
+    // 300 positions the line below (Q8_0, whose rows are the most bytes, crosses it earlier) leaves 0.4 %
+    // to the better of the two on average, 16 % at most. RQMV_MOE_DOWN_BATCH=0/1 forces either.
     const size_t blds = (size_t)nch * (size_t)(down_pitch<FMT>() + 16);
-    if (G <= 32 && blds <= 65536 && env_flag("RQMV_MOE_DOWN_BATCH", b.m >= kMoeBatchMin)) {
+    const int64_t work = (int64_t)b.m * (d.top * d.hidden + d.hidden_shared) * (d.d_model - 400);
+    if (G <= 32 && blds <= 65536 && env_flag("RQMV_MOE_DOWN_BATCH", b.m >= kMoeBatchMin && work >= (FMT == Q8_0 ? 18000000 : 25000000))) {
         const char* senv = getenv("RQMV_MOE_DOWN_SPAN");
         const int span = senv && *senv ? atoi(senv) / 32 * 32 : b.m >= 48 ? 128 : 64;
         if (span < 32) return hipErrorInvalidValue;

@@ -1,7 +1,7 @@
 """gguf_moe over batches: every position of a batch carries the bits of its own
 one-position call, in every kernel form that batches take (the router's groups
 of sixteen positions, the down product's blocks of rows with its encoded slot
-activations, the gate/up product by expert), over formats, widths that leave partial
+activations, the gate/up product by blocks of the hidden width), over formats, widths that leave partial
 row blocks and chunk rounds, a shared expert gated, ungated or absent, skewed
 routing, and activations with outliers."""
 import numpy as np
@@ -71,10 +71,31 @@ def test_gate_up_by_blocks_of_rows(gpu, case, blocks, monkeypatch):
     d, m = case[1], 18
     moe = _moe(gpu, case, seed=sum(case[1:6]))
     x = _activations(m, d, "f32", "outliers", seed=m + d)
-    y = gpu.DeviceBuffer(4 * m * d)
+    y, route = gpu.DeviceBuffer(4 * m * d), gpu.DeviceBuffer(4 * m * case[4])
     y.fill_zero()
-    moe.run_batch(gpu.DeviceBuffer.from_array(x), gpu.DTYPE_F32, m, d, y, d, None, moe.batch_workspace(m))
+    moe.run_batch(gpu.DeviceBuffer.from_array(x), gpu.DTYPE_F32, m, d, y, d, route, moe.batch_workspace(m))
     gpu.synchronize()
-    got = y.download(np.float32).reshape(m, d)
+    got, routes = y.download(np.float32).reshape(m, d), route.download(np.float32).reshape(m, case[4])
     for p in range(m):
-        assert np.array_equal(got[p].view(np.uint32), moe(x[p])[0].view(np.uint32)), (case, p)
+        y1, r1 = moe(x[p])
+        assert np.array_equal(got[p].view(np.uint32), y1.view(np.uint32)), (case, p)
+        assert np.array_equal(routes[p].view(np.uint32), r1.view(np.uint32)), (case, p)
+
+
+@pytest.mark.parametrize("case", CASES, ids=lambda c: "-".join(map(str, c)))
+@pytest.mark.parametrize("form", ["0", "1"])
+def test_down_by_blocks_of_rows(gpu, case, form, monkeypatch):
+    """The down product over whole positions and by blocks of output rows (64 rows, and
+    128 from 48 positions), at sizes that the plan leaves to one of the two."""
+    monkeypatch.setenv("RQMV_MOE_DOWN_BATCH", form)
+    d = case[1]
+    moe = _moe(gpu, case, seed=sum(case[1:6]))
+    for m in (17, 50):
+        x = _activations(m, d, "f32", "outliers", seed=m + d)
+        y = gpu.DeviceBuffer(4 * m * d)
+        y.fill_zero()
+        moe.run_batch(gpu.DeviceBuffer.from_array(x), gpu.DTYPE_F32, m, d, y, d, None, moe.batch_workspace(m))
+        gpu.synchronize()
+        got = y.download(np.float32).reshape(m, d)
+        for p in range(m):
+            assert np.array_equal(got[p].view(np.uint32), moe(x[p])[0].view(np.uint32)), (case, p)
