@@ -168,3 +168,76 @@ def test_f32_activations_near_the_largest(gpu, fmt, tile, monkeypatch):
         ref = oracle.matvec_f64(fmt, w, rows, cols, x, threads=THREADS)
         assert np.abs(ref).max() < 3e38 and np.isfinite(y).all(), (fmt, m)
         assert rel(y, ref) <= limit(cols), (fmt, m)
+
+
+@pytest.mark.parametrize("fmt", FMTS)
+@pytest.mark.parametrize("xdt", ["f16", "f32"])
+@pytest.mark.parametrize("tile", ["0", "11", "22", "14"])
+def test_non_finite_activations_stay_in_their_rows(gpu, fmt, xdt, tile, monkeypatch):
+    """More than 32 rows, a NaN in one and an infinity in another: every output of those
+    rows is non-finite, every other row keeps its bits."""
+    monkeypatch.setenv("RQMV_TILE", tile)
+    rows, cols, m = 83, 768, 70
+    W = gpu.Weight(fmt, rows, cols, synth.weights(fmt, rows, cols, seed=14))
+    dt = gpu.DTYPE_F16 if xdt == "f16" else gpu.DTYPE_F32
+    x, _ = activations(m, cols, xdt, seed=15)
+    out = []
+    for bad in (False, True):
+        if bad:
+            x = x.copy()
+            nan, inf = (0x7E00, 0x7C00) if xdt == "f16" else (np.nan, np.inf)
+            x[3, 300], x[40, 511] = nan, inf
+        yb = gpu.DeviceBuffer(4 * m * rows)
+        W.matvec(gpu.DeviceBuffer.from_array(x), dt, m, cols, yb, rows)
+        gpu.synchronize()
+        out.append(yb.download(np.float32).reshape(m, rows))
+    keep = np.ones(m, bool)
+    keep[[3, 40]] = False
+    assert np.isfinite(out[0]).all()
+    assert not np.isfinite(out[1][~keep]).any()
+    assert np.array_equal(out[0][keep].view(np.uint32), out[1][keep].view(np.uint32))
+
+
+@pytest.mark.parametrize("fmt", ["q4_k", "q8_0"])
+@pytest.mark.parametrize("xdt,tile", [("f32", "0"), ("f32", "11"), ("f16", "11")])
+def test_activations_beyond_one_launch(gpu, fmt, xdt, tile, monkeypatch):
+    """Activation rows so far apart that a launch's 32-bit offsets (4 GiB) reach only some
+    of them: the rest go in further launches."""
+    monkeypatch.setenv("RQMV_TILE", tile)
+    rows, cols, m = 40, 512, 45
+    size = 4 if xdt == "f32" else 2
+    ldx = 108_000_000 // size  # 40 rows to 4 GiB
+    w = synth.weights(fmt, rows, cols, seed=16)
+    W = gpu.Weight(fmt, rows, cols, w)
+    xh, x = activations(m, cols, xdt, seed=17)
+    big, y = gpu.DeviceBuffer(((m - 1) * ldx + cols) * size), gpu.DeviceBuffer(4 * m * rows)
+    for i in range(m):
+        row = gpu.DeviceBuffer.from_array(xh[i])
+        gpu.DeviceBuffer.copy_from(big.view(i * ldx * size, cols * size), row, cols * size)
+        gpu.synchronize()
+    W.matvec(big, gpu.DTYPE_F16 if xdt == "f16" else gpu.DTYPE_F32, m, ldx, y, rows)
+    gpu.synchronize()
+    ref = oracle.matvec_f64(fmt, w, rows, cols, x, threads=THREADS)
+    got = y.download(np.float32).reshape(m, rows)
+    for i in range(m):
+        assert rel(got[i], ref[i]) <= limit(cols), (i, rel(got[i], ref[i]))
+
+
+def test_f16_weights_beyond_one_launch(gpu):
+    """More groups of sixteen rows than a launch's y dimension holds (65,535), and a rest:
+    rows with equal activations have equal bits wherever they stand."""
+    rows, cols, base, m = 3, 64, 4096, 16 * 65535 + 37
+    w = synth.f16_weights(rows, cols, 0.05, seed=18)
+    W = gpu.Weight("f16", rows, cols, w)
+    xh = synth.activations_f16(base * cols, seed=19).reshape(base, cols)
+    x = np.concatenate([xh] * (m // base + 1))[:m]
+    y = gpu.DeviceBuffer(4 * m * rows)
+    W.matvec(gpu.DeviceBuffer.from_array(x), gpu.DTYPE_F16, m, cols, y, rows)
+    gpu.synchronize()
+    got = y.download(np.float32).reshape(m, rows)
+    ref = synth.fp16_to_f32(xh).astype(np.float64) @ synth.fp16_to_f32(w.view(np.uint16).reshape(rows, cols)).astype(np.float64).T
+    assert rel(got[:base], ref) <= limit(cols)
+    same = got.view(np.uint32) == np.concatenate([got[:base]] * (m // base + 1))[:m].view(np.uint32)
+    assert same[: m - m % 16].all()  # whole groups of sixteen; the rest runs in smaller launches
+    last = m - m % 16
+    assert rel(got[last:], np.concatenate([ref] * (m // base + 1))[last:m]) <= limit(cols)
