@@ -196,7 +196,8 @@ int rqmv_moe(const rqmv_moe_params* params, const void* x_dev, int x_dtype, floa
  * position of a step, each routed on its own): position p reads x_dev + p*ldx
  * elements and writes y_dev + p*ldy; its routing weights go to route_dev +
  * p*experts when route_dev is not NULL. The workspace holds m times
- * rqmv_moe_workspace_size bytes. Still three launches for the whole batch. */
+ * rqmv_moe_workspace_size bytes. Three launches for the whole batch, four from
+ * sixteen positions where the down product pays for one of its own. */
 int rqmv_moe_batch(const rqmv_moe_params* params, const void* x_dev, int x_dtype, int m, int64_t ldx, float* y_dev,
                    int64_t ldy, float* route_dev, void* workspace, size_t workspace_bytes, void* stream);
 

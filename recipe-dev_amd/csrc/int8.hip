@@ -456,8 +456,9 @@ __global__ __launch_bounds__(kI8Threads) void int8_slices_kernel(I8Launch p) {
 // the operations of the one-row kernel in their order. Step 32, us at 4 / 8 rows with a
 // workgroup per activation row -> four rows a workgroup: Q4_K 4096->14336 27.7 / 52.5 ->
 // 22.3 / 36.2, Q6_K 33.5 / 62.0 -> 21.2 / 32.3, Q4_0 33.2 / 61.6 -> 24.4 / 35.5; Q8_0
-// 5120x5120 14.3 / 25.9 -> 13.1 (two rows) / 20.5. Bound by the records' LDS reads and
-// the sums' round trip.
+// 5120x5120 14.3 / 25.9 -> 13.1 (two rows) / 20.5. Bound by VALU issue (0.68 of a SIMD's
+// time on Q4_K 4096->14336 at four rows) and by the records' LDS reads and the sums'
+// round trip, whose bank conflicts alone take a quarter of a CU's time.
 template <int MR>
 __device__ __forceinline__ float* stage_record_rows(const I8Launch& p, int step, uint8_t* lds) {
     q8_record_rows<MR>(p.x, p.ldx, (int)blockIdx.y * MR, p.M, p.K, step, lds, (int)threadIdx.x);

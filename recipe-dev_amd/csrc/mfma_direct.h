@@ -23,10 +23,11 @@
 // lane j of 16-lane row kq the power of row 4 kq + j, and the multiplications
 // by it take it through a row broadcast (DPP).
 //
-// Bound. The conversions of the activations, which every row tile's workgroup
-// repeats (about 45 instructions per eight values), and at few rows the round
-// trips of a wave's two or four steps; the weights' bytes take a fifth of the
-// time. Measured against the staged form this replaces (kernel us, fp32 x): Q4_K
+// Bound. VALU issue: 0.75 of a SIMD's time on Q6_K 14336->4096 at 77 rows, 0.59 on
+// Q4_K 4096x4096 at five, most of it the conversions of the activations, which every
+// row tile's workgroup repeats (about 45 instructions per eight values); at few rows
+// also the round trips of a wave's two or four steps. The weights' bytes take a fifth
+// of the time. Measured against the staged form this replaces (kernel us, fp32 x): Q4_K
 // 4096x4096 at 5 rows 83.8 -> 12.2 (780 GB/s), Q6_K 14336->4096 at 77 rows
 // 3363 -> 106 (85 TFLOP/s).
 #pragma once

@@ -25,10 +25,12 @@
 // as in mfma_direct.h, the power of two times the scale; Q4_K's minimum times the
 // block's fp32 activation sum).
 //
-// Bound. At 512 rows, VALU issue (the scaled sums, four fmas per product, and the
-// decode) beside the products with two waves per SIMD: the matrix cores are busy for
-// a fifth (fp32 x) to a third of the time. One workgroup alone takes 2-7 us a step of
-// 256 values (mfma_tile.hip), so small products are bound by the length of K.
+// Bound. With two waves per SIMD, waits: on Q4_K 4096->14336 at 512 rows, fp16 x, half
+// of the waves' time goes to loads, LDS reads and the barrier, while VALU instructions
+// issue for 0.40 of a SIMD's time, the matrix cores are busy for 0.31 and the LDS reads
+// (1 KiB per two products) take about a third of their port's. A workgroup alone takes 2 to 11
+// us a step of 256 values (mfma_tile.hip), so small products are bound by the length of
+// K.
 #pragma once
 
 #include "mfma_direct.h"

@@ -673,7 +673,8 @@ __global__ void __launch_bounds__(kMoeThreads) moe_encode_kernel(MoeDims d, MoeW
 // carries the bits of the one-position form. Workgroups go to the eight XCDs in turn;
 // an XCD takes every eighth block of rows, all positions of one block before the next,
 // so that the positions that chose an expert find its rows in the XCD's L2 or close to
-// it. Bound by VALU issue: a chunk's 32 digit dots and about 60 instructions around them.
+// it. Bound by VALU issue (all of a SIMD's time at 512 positions of the gguf_moe
+// workload): a chunk's 32 digit dots and about 60 instructions around them.
 template <int FMT>
 constexpr int down_pitch() {  // bytes of a staged chunk in LDS: lanes on consecutive chunks hit different banks
     return (Traits<FMT>::XP + Traits<FMT>::XR) * 16 + 16;
