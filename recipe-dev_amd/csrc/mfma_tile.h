@@ -17,9 +17,10 @@
 // products; both parts with the scale's sign, so that neither is larger than the
 // scale: -1 as -16 + 15 would take the rounding of sixteen times its sum, 6.6e-7
 // against 8e-8 where every scale is -1), so the matrix cores sum a whole 256-weight
-// block before fp32 arithmetic: the block's d scales the tile once per 256 weights. Q4_K's minimums are one
-// more product per 256 weights, of the eight 6-bit minimums with the eight
-// sub-blocks' activation sums, each sum as three bf16 parts (24 bits).
+// block before fp32 arithmetic: the block's d scales the tile once per 256 weights (twice
+// in short rows, kFoldWhole). Q4_K's minimums are one more product per 256 weights, of the
+// eight 6-bit minimums with the eight sub-blocks' activation sums, each sum as three bf16
+// parts (24 bits).
 // Otherwise every 32-weight block (Q6_K: each 16-weight scale group) is a product
 // of its own, scaled in fp32 into the sums (fp32 activations: high and low fp16 parts
 // as in mfma_direct.h, the power of two times the scale; Q4_K's minimum times the
@@ -66,6 +67,14 @@ __device__ __forceinline__ void nibbles_scaled(uint32_t w, hv2_t sc, hv2_t off, 
     }
 }
 
+// Rows from this length on fold whole 256-weight blocks, shorter ones halves: a chain of
+// products rounds more than the fp32 additions it replaces, which few blocks do not make
+// up for. Error against 64 bits in whole blocks / halves / a product per 32 weights, fp16
+// x: Q4_K 1.12e-7 / 0.91e-7 / 1.06e-7 and Q6_K 1.22e-7 / 0.90e-7 / 1.07e-7 at 1,024
+// columns; at 2,304 within 5 % of the last with activations of widely unlike magnitudes;
+// at 4,096 1.2e-7 in whole blocks against 2.05e-7. Halves cost up to 2 %.
+constexpr int kFoldWhole = 2560;
+
 // Waves per SIMD the registers are bounded for: the smallest tile runs two
 // workgroups per CU, the others one.
 template <int RT, int MT, int WN, int WK, bool XF32>
@@ -103,6 +112,7 @@ __global__ void __launch_bounds__(64 * WN * WK) __attribute__((amdgpu_waves_per_
     const int64_t row0 = ((int64_t)nt * WN + wave) * (16 * RT);
     uint8_t* const lds = reinterpret_cast<uint8_t*>(smem) + wk * C::LDS;  // this range's buffers
     const int nch = p.P.nch;
+    const bool halves = FOLD && RT == 1 && p.K < kFoldWhole;
     const int loads = (nch + 3) / 4, total = (loads + SPL - 1) / SPL;
     // this wave's steps (every range runs as many rounds as the longest, for the
     // barriers: those past its end compute nothing)
@@ -372,6 +382,17 @@ __global__ void __launch_bounds__(64 * WN * WK) __attribute__((amdgpu_waves_per_
                 add(MT - 1);
             }
             if constexpr (FOLD) {
+                if (wi == 0 && halves) {  // (short rows: half a block's tile at a time)
+#pragma unroll
+                    for (int t = 0; t < MT; ++t)
+#pragma unroll
+                        for (int r = 0; r < RT; ++r) {
+                            const float dd = half_lo(FMT == Q4_K ? cur[r][0].meta.x : cur[r][0].d);
+#pragma unroll
+                            for (int j = 0; j < 4; ++j) acc[r][t][j] = fmaf(dd, D[r][t][j], acc[r][t][j]);
+                            D[r][t] = z;
+                        }
+                }
                 if (wi == WPS - 1) {
                     // the 256-weight block's tile into the sums
                     b8_t Bm[FMT == Q4_K ? RT : 1];

@@ -60,19 +60,19 @@ static int fmt_slot(int fmt) { return fmt == Q4_0 ? 0 : fmt == Q4_K ? 1 : fmt ==
 
 // The best shape for a product and its estimated time (us). Rounds are those of the XCD
 // with the most workgroups (an XCD takes every eighth tile of rows). Of several, each
-// takes 1.04 of one alone, in shape 11, whose workgroups run two to a CU, 0.9 (fp16 x) or
-// 0.82. RQMV_TILE names a shape instead.
+// takes 1.04 of one alone, in shape 11, whose workgroups run two to a CU, 0.87 (fp16 x) or
+// 0.79. RQMV_TILE names a shape instead.
 static const TileShape& tile_plan(int fmt, bool f32, int64_t M, int64_t rows, int64_t cols, int cus, float* us) {
     const char* env = getenv("RQMV_TILE");
     const int want = env && *env ? atoi(env) : 0;
     const TileShape* best = nullptr;
     for (const TileShape& s : kTileShapes) {
         const float step = s.step[f32][fmt_slot(fmt)];
-        if (step == 0.f) continue;
+        if (step == 0.f || (!f32 && fmt == Q4_K && s.rt == 2 && cols < kFoldWhole)) continue;  // (that shape folds whole blocks)
         const int64_t bn = 16 * s.rt * s.wn, bm = 16 * (f32 ? s.mt / 2 : s.mt);
         const int64_t wgs = ((rows + bn - 1) / bn + 7) / 8 * 8 * ((M + bm - 1) / bm);
         const int64_t steps = ((cols + 255) / 256 + s.wk - 1) / s.wk, rounds = (wgs + cus - 1) / cus;
-        const float each = rounds == 1 ? 1.f : s.id != 11 ? 1.04f : f32 ? 0.82f : 0.9f;
+        const float each = rounds == 1 ? 1.f : s.id != 11 ? 1.04f : f32 ? 0.79f : 0.87f;
         const float t = 1.5f + (float)rounds * each * (step * (float)steps + s.round);
         if (s.id == want || (!best || (t < *us && best->id != want))) {
             best = &s;
